@@ -168,7 +168,7 @@ typedef struct rtc8x_grid {
      * a leaf (8 words) or per table entry of a lower (64 words) / upper (512 words) node, bit n of word
      * n / 64 for offset n.  A set bit on an internal table entry marks an active tile.  Decoded grids
      * carry them; the encoder writes them back, and treats NULL as every leaf voxel active and every
-     * tile inactive.  Never uploaded. */
+     * tile inactive.  Never uploaded: in a device grid the library keeps its lookup bricks here (opaque). */
     const uint64_t* leaf_masks;          /* num_leaves x 8 */
     const uint64_t* lower_masks;         /* num_lower x 64 */
     const uint64_t* upper_masks;         /* num_upper x 512 */

@@ -12,6 +12,8 @@
 //   cell_majorants  one f32 per 8^3 cell of the index bbox (largest voxel over the cell and a one-voxel rim)
 //   region_majorants one byte per region of region_cells^3 cells (quantised majorant or empty-space distance)
 //   leaf_map        one u32 per 8^3 block of the index bbox plus a one-block margin (the tree walk's result)
+//   lookup bricks   576 x 4 f32 per stored brick (the stencils of a block's voxels), and one u32 per block of
+//                   the leaf map: its brick (rtc8x_device.hpp)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -132,6 +134,83 @@ __global__ void leaf_map_kernel(const rtc8x_grid g, uint32_t* __restrict__ map)
     const uint32_t bx = (uint32_t)(r / (uint32_t)g.leaf_map_dims[1]);
     map[q] = find_leaf(g, g.leaf_map_origin[0] + 8 * (int32_t)bx, g.leaf_map_origin[1] + 8 * (int32_t)by,
                        g.leaf_map_origin[2] + 8 * (int32_t)bz);
+}
+
+// Whether block q of the leaf map (its origin in o, its entry in e) is the same tile as its seven upper
+// neighbours: its brick is then that tile's.
+__device__ __forceinline__ bool same_tile_block(const rtc8x_grid& g, size_t q, int32_t (&o)[3], uint32_t& e)
+{
+    const uint32_t dy = (uint32_t)g.leaf_map_dims[1], dz = (uint32_t)g.leaf_map_dims[2];
+    o[0] = g.leaf_map_origin[0] + 8 * (int32_t)(q / ((size_t)dy * dz));
+    o[1] = g.leaf_map_origin[1] + 8 * (int32_t)((q / dz) % dy);
+    o[2] = g.leaf_map_origin[2] + 8 * (int32_t)(q % dz);
+    e = g.leaf_map[q];
+    bool same = (e & RTC8X_TILE_BIT) != 0u;
+    for (int32_t t = 1; t < 8 && same; ++t)
+        same = block_entry(g, o[0] + 8 * (t >> 2), o[1] + 8 * ((t >> 1) & 1), o[2] + 8 * (t & 1)) == e;
+    return same;
+}
+
+// Blocks with a brick of their own per 256-lane workgroup.
+__global__ __launch_bounds__(256) void brick_count_kernel(const rtc8x_grid g, size_t n, uint32_t* __restrict__ sums)
+{
+    __shared__ uint32_t part[4];
+    const size_t q = (size_t)blockIdx.x * 256 + threadIdx.x;
+    int32_t o[3];
+    uint32_t e;
+    const uint64_t own = __ballot(q < n && !same_tile_block(g, q, o, e));
+    if ((threadIdx.x & 63u) == 0) part[threadIdx.x >> 6] = (uint32_t)__popcll(own);
+    __syncthreads();
+    if (threadIdx.x == 0) sums[blockIdx.x] = part[0] + part[1] + part[2] + part[3];
+}
+
+// The map's entries: the first quad of each block's brick.  Two quads per tile value come first, then the
+// blocks' own bricks in block order (base: the exclusive scan of the counts above).
+__global__ __launch_bounds__(256) void brick_map_kernel(const rtc8x_grid g, size_t n, uint32_t num_tiles,
+                                                        const uint32_t* __restrict__ base, uint32_t* __restrict__ map,
+                                                        uint32_t* __restrict__ block_of)
+{
+    __shared__ uint32_t part[4];
+    const size_t q = (size_t)blockIdx.x * 256 + threadIdx.x;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    int32_t o[3];
+    uint32_t e = 0;
+    const bool own = q < n && !same_tile_block(g, q, o, e);
+    const uint64_t owners = __ballot(own);
+    if (lane == 0) part[wave] = (uint32_t)__popcll(owners);
+    __syncthreads();
+    uint32_t r = base[blockIdx.x] + (uint32_t)__popcll(owners & ((1ull << lane) - 1ull));
+    for (uint32_t w = 0; w < wave; ++w) r += part[w];
+    if (own) block_of[r] = (uint32_t)q;
+    if (q < n) map[q] = own ? 2 * num_tiles + r * kBrickQuads : kSharedBrick | 2 * (e & ~RTC8X_TILE_BIT);
+}
+
+// One workgroup per brick, and behind them one lane per tile value.
+__global__ __launch_bounds__(256) void brick_fill_kernel(const rtc8x_grid g, uint32_t num_bricks, uint32_t num_tiles,
+                                                         const uint32_t* __restrict__ block_of, float4* __restrict__ bricks)
+{
+    if (blockIdx.x >= num_bricks) {
+        const uint32_t t = (blockIdx.x - num_bricks) * 256 + threadIdx.x;
+        if (t >= num_tiles) return;
+        const float v = g.tile_values[t];
+        bricks[2 * (size_t)t] = bricks[2 * (size_t)t + 1] = make_float4(v, v, v, v);
+        return;
+    }
+    // the block's voxels and one layer more on the upper faces
+    __shared__ float vox[9][9][9];
+    int32_t o[3];
+    uint32_t e;
+    (void)same_tile_block(g, block_of[blockIdx.x], o, e);
+    for (uint32_t v = threadIdx.x; v < 729; v += 256) {
+        const int32_t i = o[0] + (int32_t)(v / 81), j = o[1] + (int32_t)(v / 9 % 9), k = o[2] + (int32_t)(v % 9);
+        (&vox[0][0][0])[v] = *voxel_ptr(g, block_entry(g, i, j, k), i, j, k);
+    }
+    __syncthreads();
+    float4* out = bricks + 2 * (size_t)num_tiles + (size_t)blockIdx.x * kBrickQuads;
+    for (uint32_t q = threadIdx.x; q < kBrickQuads; q += 256) {
+        const uint32_t x = q / 72, y = q / 9 % 8, z = q % 9;
+        out[q] = make_float4(vox[x][y][z], vox[x][y + 1][z], vox[x + 1][y][z], vox[x + 1][y + 1][z]);
+    }
 }
 
 // One wavefront per 8^3 cell c (cell_origin + 8c): the largest voxel value, through the tree (leaves,
@@ -315,6 +394,69 @@ rtc8x_status build_leaf_map(rtc8x_grid& g, hipStream_t s)
     return RTC8X_OK;
 }
 
+// Frees what it holds unless it was released to the grid.
+template <typename T>
+struct DeviceArray {
+    T* p = nullptr;
+    ~DeviceArray()
+    {
+        if (p) (void)hipFree(p);
+    }
+    bool alloc(size_t count)
+    {
+        if (hipMalloc((void**)&p, std::max<size_t>(count, 1) * sizeof(T)) == hipSuccess) return true;
+        (void)hipGetLastError();
+        p = nullptr;
+        return false;
+    }
+    T* release()
+    {
+        T* r = p;
+        p = nullptr;
+        return r;
+    }
+};
+
+// The lookup bricks of a grid with a leaf map (rtc8x_device.hpp); num_tiles tile values.  Grids whose bricks
+// would take 2^31 quads (32 GiB) or more, or do not fit the device, go without: lookups then walk the tree.
+rtc8x_status build_bricks(rtc8x_grid& g, uint32_t num_tiles, hipStream_t s)
+{
+    g.leaf_masks = g.lower_masks = g.upper_masks = nullptr;
+    const uint64_t d0 = (uint64_t)g.leaf_map_dims[0], d1 = (uint64_t)g.leaf_map_dims[1], d2 = (uint64_t)g.leaf_map_dims[2];
+    if (!g.leaf_map || d0 * d1 >= (1u << 24) || d2 >= (1u << 24)) return RTC8X_OK;  // the lookup's 24-bit products
+    const size_t n = (size_t)(d0 * d1 * d2);
+    const uint32_t groups = (uint32_t)((n + 255) / 256);
+    DeviceArray<uint32_t> sums, map, block_of;
+    DeviceArray<float4> bricks;
+    if (!sums.alloc(groups) || !map.alloc(n)) return RTC8X_OK;
+    hipLaunchKernelGGL(dev::brick_count_kernel, dim3(groups), dim3(256), 0, s, g, n, sums.p);
+    RTC8X_HIP(hipGetLastError());
+    std::vector<uint32_t> base(groups);
+    RTC8X_HIP(hipMemcpyAsync(base.data(), sums.p, groups * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    RTC8X_HIP(hipStreamSynchronize(s));
+    uint64_t own = 0;
+    for (uint32_t& b : base) {
+        const uint32_t c = b;
+        b = (uint32_t)own;
+        own += c;
+    }
+    const uint64_t quads = 2 * (uint64_t)num_tiles + own * dev::kBrickQuads;
+    if (quads >= dev::kSharedBrick) return RTC8X_OK;
+    if (!block_of.alloc(own) || !bricks.alloc(quads)) return RTC8X_OK;
+    RTC8X_HIP(hipMemcpyAsync(sums.p, base.data(), groups * sizeof(uint32_t), hipMemcpyHostToDevice, s));
+    hipLaunchKernelGGL(dev::brick_map_kernel, dim3(groups), dim3(256), 0, s, g, n, num_tiles, (const uint32_t*)sums.p, map.p,
+                       block_of.p);
+    RTC8X_HIP(hipGetLastError());
+    hipLaunchKernelGGL(dev::brick_fill_kernel, dim3((uint32_t)own + (num_tiles + 255) / 256), dim3(256), 0, s, g,
+                       (uint32_t)own, num_tiles, (const uint32_t*)block_of.p, bricks.p);
+    RTC8X_HIP(hipGetLastError());
+    RTC8X_HIP(hipStreamSynchronize(s));
+    g.lower_masks = reinterpret_cast<const uint64_t*>(bricks.release());
+    g.leaf_masks = reinterpret_cast<const uint64_t*>(map.release());
+    g.upper_masks = reinterpret_cast<const uint64_t*>((uintptr_t)dev::brick_tag(g.lower_masks, g.leaf_masks));
+    return RTC8X_OK;
+}
+
 // The cell majorants of a device grid (cell grid over the index bbox, from cell_max_kernel) and its region
 // table (region_cells as region_majorants takes it).  Grids without leaves, or whose index bbox spans more
 // than 2^26 cells, get neither (local-majorant tracking then refuses them).
@@ -403,6 +545,10 @@ try {
     RTC8X_REQUIRE(g != nullptr, "rtc8x_grid_destroy: grid is NULL");
     const void* ptrs[] = {g->root_tiles, g->upper_tables, g->lower_tables, g->leaf_values,     g->tile_values,
                           g->leaf_origins, g->cell_majorants, g->leaf_map,    g->region_majorants};
+    if (dev::brick_tagged(*g)) {
+        RTC8X_HIP(hipFree(const_cast<uint64_t*>(g->lower_masks)));
+        RTC8X_HIP(hipFree(const_cast<uint64_t*>(g->leaf_masks)));
+    }
     for (const void* p : ptrs)
         if (p) RTC8X_HIP(hipFree(const_cast<void*>(p)));
     std::memset(g, 0, sizeof(*g));
@@ -552,6 +698,7 @@ try {
     RTC8X_HIP(hipGetLastError());
     RTC8X_HIP(hipStreamSynchronize(s));
     RTC8X_TRY(build_leaf_map(g, s));
+    RTC8X_TRY(build_bricks(g, 1, s));
     RTC8X_TRY(build_majorant_tables(g, 0, s));
     *out = g;
     return RTC8X_OK;
@@ -644,7 +791,10 @@ rtc8x_status upload_host_grid(const rtc8x_grid* h, rtc8x_grid* out, bool keep_ma
     g.region_majorants = nullptr;
     g.leaf_map = nullptr;
     g.leaf_masks = g.lower_masks = g.upper_masks = nullptr;  // host-side activity is not uploaded
-    if (h->num_root_tiles > 0 && h->num_leaves > 0) RTC8X_TRY(build_leaf_map(g, nullptr));
+    if (h->num_root_tiles > 0 && h->num_leaves > 0) {
+        RTC8X_TRY(build_leaf_map(g, nullptr));
+        RTC8X_TRY(build_bricks(g, num_tiles_values, nullptr));
+    }
     RTC8X_TRY(build_majorant_tables(g, 0, nullptr));
     *out = g;
     return RTC8X_OK;
