@@ -103,9 +103,7 @@ void march_probe_kernel(const rtc8x_frame_params p, dev::V3 light, uint32_t spp,
     const float coeff = p.density_coeff;
     const float trace_len = 2.0f * p.world_radius;
     dev::Medium med;
-    med.coeff = coeff;
-    med.majorant = maj;
-    med.lookups = 0;
+    med.init(p.grid, coeff);
     dev::Seg<RTC8X_TRACKING_LOCAL_MAJORANT> sg;
     dev::Pcg rng;
     rng.state = 0;
@@ -173,9 +171,9 @@ void march_probe_kernel(const rtc8x_frame_params p, dev::V3 light, uint32_t spp,
                 const float sig = dev::sample_density(p.grid, med, sg.o, sg.d, sg.t);
                 ++looked;
                 if (mode == 1) {
-                    if (sg.after_track(rng, sig, mu)) event = 1;
+                    if (sg.after_track(med, rng, sig, mu)) event = 1;
                 } else {
-                    sg.after_shadow(rng, sig, mu, vis);
+                    sg.after_shadow(med, rng, sig, mu, vis);
                 }
             } else if (r == dev::kAdvanceEnd) {
                 event = 2;
@@ -187,8 +185,8 @@ void march_probe_kernel(const rtc8x_frame_params p, dev::V3 light, uint32_t spp,
             // two tentative collisions (a collision past the segment's end is looked up at the current
             // position, as the tracer does); a tracking segment stops at the first real one
             float tk[2], tl[2], u[2];
-            tk[0] = t - rtc8x_logf(1.0f - rng.uni()) / maj;
-            tk[1] = tk[0] - rtc8x_logf(1.0f - rng.uni()) / maj;
+            tk[0] = t + med.over(dev::neg_log_1m(rng.uni()), maj);
+            tk[1] = tk[0] + med.over(dev::neg_log_1m(rng.uni()), maj);
             u[0] = rng.uni();
             u[1] = rng.uni();
             tl[0] = tk[0] > t1 ? t : tk[0];
@@ -203,9 +201,9 @@ void march_probe_kernel(const rtc8x_frame_params p, dev::V3 light, uint32_t spp,
                 ++looked;
                 t = tk[k];
                 if (mode == 1) {
-                    if (u[k] < sig[k] / maj) event = 1;
+                    if (u[k] < med.over(sig[k], maj)) event = 1;
                 } else {
-                    vis *= 1.0f - sig[k] / maj;
+                    vis *= 1.0f - med.over(sig[k], maj);
                 }
             }
         }

@@ -1,6 +1,7 @@
 // rtc8x_trace.hip -- the path-tracing launch: the three OptiX ray-generation programs
 // (pathTrace, generateTrainingData, pathTraceWithNRC; renderer/gpu_kernels/optix_pathtracing_kernels.cu
-// :31-448) for volume-only scenes, as one persistent per-lookup state machine.
+// :31-448) for volume-only scenes.  The full-image launches run in rtc8x_slots.hpp; the training launch and
+// the batched launches run here, as one persistent per-lookup state machine.
 //
 // A lane owns one pixel at a time (all of its samples, so the pixel's PCG stream is consumed in the
 // reference's order) and steps its path through free-flight tracking towards the next scattering
@@ -35,6 +36,7 @@ constexpr uint32_t kSpeculate = 2;
 constexpr uint32_t kCoopIdle = 48;
 constexpr uint32_t kTrainSpreadLanes = 64 - kCoopIdle;  // paths per wavefront of a spread training launch
 constexpr uint32_t kCoopLocalPaths = 2;  // at most this many stepping lanes for the local walk's cooperative tail
+constexpr uint32_t kCoopClaim = 4;  // a wavefront's claim of at most this many global segments is taken cooperatively
 constexpr uint32_t kCounterSlots = 1024;
 constexpr uint32_t kMaxBatch = 16;  // instances of one batched launch
 __device__ uint32_t g_work_counter[kCounterSlots];
@@ -60,14 +62,14 @@ struct Seg<RTC8X_TRACKING_GLOBAL_MAJORANT> {
     }
     __device__ __forceinline__ bool advance(const rtc8x_grid&, const Medium& m, Pcg& rng, float& mu, const uint8_t*)
     {
-        t += -rtc8x_logf(1.0f - rng.uni()) / m.majorant;
+        t += m.over(neg_log_1m(rng.uni()), m.majorant);
         if (t > t1) return false;
         mu = m.majorant;
         return true;
     }
     // returns true when the tentative collision is real
-    __device__ __forceinline__ bool after_track(Pcg& rng, float sigma, float mu) { return rng.uni() < sigma / mu; }
-    __device__ __forceinline__ void after_shadow(Pcg&, float sigma, float mu, float& vis) { vis *= 1.0f - sigma / mu; }
+    __device__ __forceinline__ bool after_track(const Medium& m, Pcg& rng, float sigma, float mu) { return rng.uni() < m.over(sigma, mu); }
+    __device__ __forceinline__ void after_shadow(const Medium& m, Pcg&, float sigma, float mu, float& vis) { vis *= 1.0f - m.over(sigma, mu); }
 };
 
 enum : uint32_t {
@@ -129,7 +131,7 @@ __device__ __forceinline__ void speculate_global(const rtc8x_grid& g, Medium& me
         ua[k] = 0.0f;
         st_after[k] = 0;
         if (!ended) {
-            t += -rtc8x_logf(1.0f - r.uni()) / med.majorant;
+            t += med.over(neg_log_1m(r.uni()), med.majorant);
             if (t > sg.t1) {
                 ended = true;
                 st_end = r.state;
@@ -151,13 +153,13 @@ __device__ __forceinline__ void speculate_global(const rtc8x_grid& g, Medium& me
         if (!accepted && k < n) {
             med.lookups++;
             if (track) {
-                if (ua[k] < sig[k] / med.majorant) {
+                if (ua[k] < med.over(sig[k], med.majorant)) {
                     accepted = true;
                     t_acc = tk[k];
                     st_acc = st_after[k];
                 }
             } else {
-                L.vis *= 1.0f - sig[k] / med.majorant;
+                L.vis *= 1.0f - med.over(sig[k], med.majorant);
             }
         }
     }
@@ -260,7 +262,7 @@ __device__ __forceinline__ void coop_segments(const rtc8x_grid& g, Medium& med, 
             const uint64_t st_step = r.state;  // after the step's draw
             const float ua = track ? r.uni() : 0.0f;
             const uint64_t st_after = r.state;
-            const float dj = -rtc8x_logf(1.0f - u) / maj;
+            const float dj = med.over(neg_log_1m(u), maj);
             // t after collision j, summed in order; the segment ends at the first collision past t1
             float tj = INFINITY, run = t;
             uint32_t e = 64;
@@ -276,7 +278,7 @@ __device__ __forceinline__ void coop_segments(const rtc8x_grid& g, Medium& med, 
             float sig = 0.0f;
             if (valid) sig = density_at(g, med.coeff, o, d, tj);
             if (track) {
-                const uint64_t acc = __ballot(valid && ua < sig / maj);
+                const uint64_t acc = __ballot(valid && ua < med.over(sig, maj));
                 if (acc) {
                     const uint32_t a = (uint32_t)__ffsll((long long)acc) - 1u;
                     looked += a + 1;
@@ -292,7 +294,7 @@ __device__ __forceinline__ void coop_segments(const rtc8x_grid& g, Medium& med, 
                     break;
                 }
             } else {
-                const float f = 1.0f - sig / maj;
+                const float f = 1.0f - med.over(sig, maj);
                 for (uint32_t i = 0; i < e; ++i) vis *= lane_f(f, i);
                 looked += e;
                 if (e < 64) {
@@ -368,7 +370,7 @@ __device__ __forceinline__ void coop_segments_local(const rtc8x_grid& g, Medium&
             uint64_t st_acc = 0;  // after the collision's acceptance number
 #pragma unroll 1
             for (uint32_t i = 0; i <= lane; ++i) {
-                if (i > 0) c.tau = -rtc8x_logf(1.0f - r.uni());
+                if (i > 0) c.tau = neg_log_1m(r.uni());
                 int res;
                 do {
                     res = c.advance(g, med, r, mu, table);
@@ -385,7 +387,7 @@ __device__ __forceinline__ void coop_segments_local(const rtc8x_grid& g, Medium&
             const float sig = valid ? density_at(g, med.coeff, c.o, c.d, c.t) : 0.0f;
             const uint32_t e = (uint32_t)__popcll(__ballot(valid));  // the valid lanes are 0 .. e-1
             if (track) {
-                const uint64_t acc = __ballot(valid && ua < sig / mu);
+                const uint64_t acc = __ballot(valid && ua < med.over(sig, mu));
                 if (acc) {
                     const uint32_t a = (uint32_t)__ffsll((long long)acc) - 1u;
                     looked += a + 1;
@@ -395,7 +397,7 @@ __device__ __forceinline__ void coop_segments_local(const rtc8x_grid& g, Medium&
                     break;
                 }
             } else {
-                const float f = valid ? 1.0f - sig / mu : 1.0f;
+                const float f = valid ? 1.0f - med.over(sig, mu) : 1.0f;
                 for (uint32_t i = 0; i < e; ++i) vis *= lane_f(f, i);
             }
             looked += e;
@@ -408,7 +410,7 @@ __device__ __forceinline__ void coop_segments_local(const rtc8x_grid& g, Medium&
             w = take(c, 63);
             Pcg rn;
             rn.state = lane_u64(track ? st_acc : r.state, 63);
-            w.tau = -rtc8x_logf(1.0f - rn.uni());
+            w.tau = neg_log_1m(rn.uni());
             st = rn.state;
         }
         if (lane == src) {
@@ -490,9 +492,7 @@ __device__ __forceinline__ void trace_body(const rtc8x_frame_params& p, uint32_t
     const float prob_env = (p.sun.enabled && p.env.kind != RTC8X_ENV_NONE) ? 1.0f - p.sun.select_prob : 1.0f;
 
     Medium med;
-    med.coeff = p.density_coeff;
-    med.majorant = p.density_coeff * p.grid.max_value;
-    med.lookups = 0;
+    med.init(p.grid, p.density_coeff);
     uint32_t paths = 0, vertices = 0, scatters = 0;
 
     Lane L;
@@ -936,25 +936,25 @@ __device__ __forceinline__ void trace_body(const rtc8x_frame_params& p, uint32_t
                     u_first = L.rng.uni();
                     st_first = L.rng.state;
                 }
-                sg.tau = -rtc8x_logf(1.0f - L.rng.uni());
+                sg.tau = neg_log_1m(L.rng.uni());
                 float mu_second = 0.0f;
                 const int r2 = sg.advance(p.grid, med, L.rng, mu_second, region_table);
                 const float tk[2] = {t_first, r2 == kAdvanceCollision ? sg.t : t_first};
                 float sig[2];
                 density_batch<2>(p.grid, med.coeff, sg.o, sg.d, tk, sig);
                 med.lookups++;
-                if (track && u_first < sig[0] / mu_first) {
+                if (track && u_first < med.over(sig[0], mu_first)) {
                     sg.t = t_first;
                     L.rng.state = st_first;
                     L.mode = kModeScatter;
                 } else {
-                    if (!track) L.vis *= 1.0f - sig[0] / mu_first;
+                    if (!track) L.vis *= 1.0f - med.over(sig[0], mu_first);
                     if (r2 == kAdvanceCollision) {
                         med.lookups++;
                         if (track) {
-                            if (sg.after_track(L.rng, sig[1], mu_second)) L.mode = kModeScatter;
+                            if (sg.after_track(med, L.rng, sig[1], mu_second)) L.mode = kModeScatter;
                         } else {
-                            sg.after_shadow(L.rng, sig[1], mu_second, L.vis);
+                            sg.after_shadow(med, L.rng, sig[1], mu_second, L.vis);
                         }
                     } else if (r2 == kAdvanceEnd) {
                         L.mode = track ? kModeEscape : kModeNeeDone;
@@ -982,6 +982,14 @@ __device__ __forceinline__ void trace_body(const rtc8x_frame_params& p, uint32_t
         }
     }
 }
+
+}  // namespace dev
+}  // namespace rtc8x
+
+#include "rtc8x_slots.hpp"
+
+namespace rtc8x {
+namespace dev {
 
 // Work counters of a launch: a block of kMaxBatch slots, taken in turn by successive launches. Launches
 // on different streams count in different slots as long as fewer than kCounterSlots / kMaxBatch of
@@ -1417,6 +1425,41 @@ hipError_t launch(const rtc8x_frame_params& p, uint32_t w, uint32_t h, uint32_t 
     return hipGetLastError();
 }
 
+// Wavefronts of a workgroup: 16 fill the SIMDs' registers (12: 28.6 ms per local-majorant frame of the 512^3
+// cloud at 1080p, 16: 24.9; 31.1 and 30.2 global).  An image whose paths fill no more than eight takes eight:
+// the others would only look for work (256 x 256, 4 samples: 0.71 ms with 8, 0.74 with 6, 0.75 with 12, 0.85
+// with 16 wavefronts).
+constexpr uint32_t kSlotWaves = 16, kSlotWavesFew = 8;
+template <int ENTRY, int TRACKING, uint32_t REGION_BYTES>
+hipError_t launch_slots(const rtc8x_frame_params& p, uint32_t num_samples, hipStream_t stream)
+{
+    const uint32_t ctr = take_counter_slots();
+    int dev = 0, cus = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(reset_counter_kernel, dim3(1), dim3(1), 0, stream, ctr);
+    const uint64_t share = ((uint64_t)p.image_width * p.image_height + cus - 1) / cus;
+    const uint32_t waves = share <= 64 * kSlotWavesFew ? kSlotWavesFew : kSlotWaves;
+    hipLaunchKernelGGL((slots_kernel<ENTRY, TRACKING, REGION_BYTES, kSlotWaves>), dim3((uint32_t)cus), dim3(64 * waves), 0,
+                       stream, p, p.image_width, p.image_height, num_samples, ctr);
+    return hipGetLastError();
+}
+
+// A small region table leaves room for more slots.
+constexpr uint32_t kSmallRegions = 8192;
+template <int ENTRY>
+hipError_t launch_slots_tracking(const rtc8x_frame_params& p, uint32_t num_samples, hipStream_t stream)
+{
+    if (p.tracking != RTC8X_TRACKING_LOCAL_MAJORANT)
+        return launch_slots<ENTRY, RTC8X_TRACKING_GLOBAL_MAJORANT, 0>(p, num_samples, stream);
+    const uint32_t regions = ((uint32_t)p.grid.region_dims[0] * (uint32_t)p.grid.region_dims[1] * (uint32_t)p.grid.region_dims[2] + 15u) & ~15u;
+    if (regions <= kSmallRegions)
+        return launch_slots<ENTRY, RTC8X_TRACKING_LOCAL_MAJORANT, kSmallRegions>(p, num_samples, stream);
+    return launch_slots<ENTRY, RTC8X_TRACKING_LOCAL_MAJORANT, RTC8X_MAX_REGIONS>(p, num_samples, stream);
+}
+
 // One persistent launch over several instances; shares[i] is instance i's part of the device's
 // workgroups (each gets at least one).
 template <int ENTRY, int TRACKING>
@@ -1637,8 +1680,7 @@ try {
     }
     hipStream_t s = (hipStream_t)stream;
     if (entry == RTC8X_ENTRY_PATH_TRACE) {
-        RTC8X_HIP((dev::launch_tracking<RTC8X_ENTRY_PATH_TRACE>(p, p.image_width, p.image_height, num_samples,
-                                                                        nullptr, nullptr, s)));
+        RTC8X_HIP(dev::launch_slots_tracking<RTC8X_ENTRY_PATH_TRACE>(p, num_samples, s));
         return RTC8X_OK;
     }
     const rtc8x_nrc_buffers& nb = p.nrc;
@@ -1646,8 +1688,7 @@ try {
                   "rtc8x_trace: NRC buffers missing");
     if (entry == RTC8X_ENTRY_PATH_TRACE_WITH_NRC) {
         RTC8X_REQUIRE(nb.inference_terminals && nb.per_frame_contribution, "rtc8x_trace: NRC buffers missing");
-        RTC8X_HIP((dev::launch_tracking<RTC8X_ENTRY_PATH_TRACE_WITH_NRC>(p, p.image_width, p.image_height, num_samples,
-                                                                                 nullptr, nullptr, s)));
+        RTC8X_HIP(dev::launch_slots_tracking<RTC8X_ENTRY_PATH_TRACE_WITH_NRC>(p, num_samples, s));
         return RTC8X_OK;
     }
     // GENERATE_TRAINING_DATA: the launch size lives on the device (prepareNRC writes it); the kernels read

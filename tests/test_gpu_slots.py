@@ -1,0 +1,46 @@
+"""GPU parity of the slot scheduler with the FP32 oracle, bit for bit, at the sizes where it changes its
+ways: one pixel, fewer pixels than workgroups, ragged images dealt out to the workgroups, and more pixels
+than all slots hold (the work counter, with and without a work order); both trackers, a region table small
+and large, a majorant beyond the range of the fast division."""
+import numpy as np
+import pytest
+
+from oracle_lib import trace_parity_case
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(res, pixels, spp):
+    assert res["rng_equal"] and res["vertices_equal"]
+    assert np.array_equal(res["gpu_accum"].view(np.uint64), res["cpu_accum"].view(np.uint64))
+    assert res["paths"] == pixels * spp
+    assert res["lookups"] == int(res["cpu_stats"][2])
+
+
+@pytest.mark.parametrize("tracking", [0, 1])
+@pytest.mark.parametrize("width,height,spp", [(1, 1, 3), (9, 3, 2), (157, 83, 1)])
+def test_few_pixels(width, height, spp, tracking):
+    _check(trace_parity_case("dense128", width=width, height=height, spp=spp, tracking=tracking, fbm_resolution=64),
+           width * height, spp)
+
+
+@pytest.mark.parametrize("tracking,config", [(0, "sparse512"), (1, "sparse512"), (1, "dense128")])
+def test_more_pixels_than_slots(tracking, config):
+    """Two launches: the second takes the pixels in the work order of the first."""
+    w, h = 701, 547
+    res = trace_parity_case(config, width=w, height=h, spp=2, tracking=tracking, fbm_resolution=64, samples_per_launch=1,
+                            env_kind="constant", max_path_length=24)
+    _check(res, w * h, 2)
+
+
+@pytest.mark.parametrize("region_cells", [1, 2])
+def test_large_region_table(region_cells):
+    """32,768 regions (the largest table) and 4,096 on the 256^3 cloud."""
+    _check(trace_parity_case("sparse512", width=96, height=54, spp=2, tracking=1, fbm_resolution=256, env_kind="constant",
+                             region_cells=region_cells), 96 * 54, 2)
+
+
+@pytest.mark.parametrize("tracking", [0, 1])
+def test_majorant_below_the_fast_divisions_range(tracking):
+    _check(trace_parity_case("dense128", width=40, height=24, spp=2, tracking=tracking, fbm_resolution=64,
+                             density_coeff=2.0 ** -42), 40 * 24, 2)
