@@ -345,14 +345,14 @@ typedef struct rtc8x_env_light {
     /* Two-level alias tables (RegularConstantContinuousDistribution2D with alias tables,
      * common_renderer_types.h:338-418): a marginal over the `height` rows and one conditional
      * table per row over `width` texels.  Weights are the importance-map mip-0 values
-     * (luminance * pi/2 * sin(theta)); the tables are built on the host in FP64. */
+     * (luminance * pi/2 * sin(theta)); the tables are built in FP64. */
     float alias_integral;        /* sum of all weights */
     const rtc8x_alias_entry* alias_rows;   /* height entries */
     const rtc8x_alias_entry* alias_cols;   /* height * width entries */
     const float* alias_weights;  /* width*height texel weights */
 } rtc8x_env_light;
 
-/* Builds the two-level alias tables for `env` from its texels (FP64 on the host; device buffers are
+/* Builds the two-level alias tables for `env` from its texels (FP64 on the device; device buffers are
  * library-owned and released with rtc8x_env_release).  Also builds the hierarchical importance map
  * (mips) on the device as computeImportanceMap does (compute_light_probs.cu:161-211). */
 rtc8x_status rtc8x_env_build_sampler(rtc8x_env_light* env, void* stream);

@@ -142,3 +142,55 @@ def test_importance_map_at_the_benchmark_sky_size_equals_the_oracle():
         assert he.map_integral > 0
     finally:
         ds.close()
+
+
+def _vose(w):
+    """Vose's method as its definition runs it: stacks in index order, their tops paired."""
+    n, total = len(w), 0.0
+    for x in w:
+        total += x
+    scaled = [x * float(n) / total if total > 0.0 else 1.0 for x in w]
+    small = [i for i in range(n) if scaled[i] < 1.0]
+    large = [i for i in range(n) if not scaled[i] < 1.0]
+    second, first = np.arange(n, dtype=np.uint32), np.ones(n, np.float32)
+    while small and large:
+        s, l = small.pop(), large[-1]
+        first[s], second[s] = scaled[s], l
+        scaled[l] = (scaled[l] + scaled[s]) - 1.0
+        if scaled[l] < 1.0:
+            small.append(large.pop())
+    return total, second, first
+
+
+@pytest.mark.parametrize("w,h", [(1, 1), (2, 1), (64, 64), (65, 33), (130, 70), (16384, 3)])
+def test_alias_tables_equal_the_serial_method(w, h):
+    """Every entry of the tables built on the device is that of the serial method in FP64: one entry, whole and
+    broken batches of 64, rows of equal and of zero weights, the widest texture."""
+    from rtcamp8_amd import _abi
+    from rtcamp8_amd._lib import call
+    from rtcamp8_amd.device import DeviceBuffer, download_ptr
+
+    rng = np.random.default_rng(w + h)
+    tex = np.exp(rng.normal(0.0, 2.0, (h, w, 4))).astype(np.float32)
+    if h > 5:
+        tex[5] = 0.0
+        tex[3] = 1.0
+        tex[:, ::3] = 0.0
+    d = DeviceBuffer.from_array(tex)
+    env = _abi.EnvLight()
+    env.kind, env.width, env.height, env.texels = _abi.ENV_LATLONG, w, h, d.ptr
+    call("rtc8x_env_build_sampler", C.byref(env), None)
+    try:
+        weights = download_ptr(env.alias_weights, np.float32, w * h).reshape(h, w)
+        cols = download_ptr(env.alias_cols, np.uint32, 2 * w * h).reshape(h, w, 2)
+        rows = download_ptr(env.alias_rows, np.uint32, 2 * h).reshape(h, 2)
+        sums = []
+        for y in range(h):
+            total, second, first = _vose([float(x) for x in weights[y]])
+            sums.append(total)
+            assert np.array_equal(second, cols[y, :, 0]) and np.array_equal(first.view(np.uint32), cols[y, :, 1]), y
+        total, second, first = _vose(sums)
+        assert np.array_equal(second, rows[:, 0]) and np.array_equal(first.view(np.uint32), rows[:, 1])
+        assert env.alias_integral == np.float32(total)
+    finally:
+        call("rtc8x_env_release", C.byref(env))
