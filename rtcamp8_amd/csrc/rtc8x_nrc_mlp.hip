@@ -117,6 +117,11 @@ inline uint32_t hash_geometry(HashGeom* g)
     return off;
 }
 
+__device__ __forceinline__ uint32_t level_entries(const HashGeom& gm, uint32_t l, uint32_t p_grid)
+{
+    return ((l + 1 < kHashLevels ? gm.offset[l + 1] : p_grid) - gm.offset[l]) / RTC8X_NRC_HASH_FEATURES;
+}
+
 // Corner c (bit 0: x, 1: y, 2: z) of level l for the clamped position p: table float index and weight.
 __device__ __forceinline__ void hash_corner(const HashGeom& gm, uint32_t l, const uint32_t gi[3], const float f[3],
                                             uint32_t c, uint32_t& idx, float& w)
@@ -477,6 +482,221 @@ __global__ __launch_bounds__(64 * WPB, WPB == 1 ? 1 : 3) void forward_kernel(con
     if (lane == 0) loss_part[blockIdx.x * WPB + wave] = loss;
 }
 
+// ---------------------------------------------------------------- hash-grid inference from LDS
+// The hash encoding's gathers -- 16 levels x 8 corners of 8 bytes per query, in tables of 256 KB a level -- go
+// through the L1 one cache line per lane: 268 M of them for 2^21 queries, 0.80 ms, five times what the network
+// takes.  A level's table of one feature is 128 KB and fits a CU's LDS.  Here a workgroup per CU holds 4,096
+// queries (eight per lane), and takes the 32 planes (level, feature) one after the other: stages the plane,
+// and gathers every query's eight corners from it.  The features stay in registers (16 pairs per query); then
+// the wavefronts run the network on their queries, 64 at a time, in the same LDS.  The sums are hash_level's,
+// in its order.
+//
+// The planes come from memory to LDS directly (through registers, 8 loads in flight: 117 us for a tile's 32
+// planes instead of 66; with all 16 in flight the features spilled).
+//
+// The queries are the live ones of the inference: a workgroup takes every gridDim-th block of 512 slots,
+// compacts the slots with a query into a list and runs each full tile of it, so slots without a query cost
+// their flag only.
+constexpr uint32_t kPlaneWaves = 8, kPlaneThreads = 64 * kPlaneWaves, kPlaneQ = 8, kPlaneTile = kPlaneThreads * kPlaneQ;
+typedef uint32_t u16v __attribute__((ext_vector_type(16)));
+
+template <typename T>
+__device__ __forceinline__ uint32_t pack_pair(float a, float b)
+{
+    const T v[2] = {(T)a, (T)b};
+    uint32_t r;
+    __builtin_memcpy(&r, v, sizeof(r));
+    return r;
+}
+
+// One feature of one level: the trilinear sum over the cell's corners, from the staged plane (hash_corner's
+// entries; stride != 0 for a dense level).  Entries are carried as byte offsets: the products and XORs of the
+// hash are taken on numbers shifted by two.
+__device__ __forceinline__ float plane_sum(const float* __restrict__ plane, const float (&p)[3], float scale, uint32_t stride)
+{
+    float f[3];
+    uint32_t g[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const float pos = p[d] * scale + 0.5f;
+        const float fl = floorf(pos);
+        f[d] = pos - fl;
+        g[d] = (uint32_t)fl;
+    }
+    const uint32_t my = (stride ? stride : 2654435761u) * 4u, mz = (stride ? stride * stride : 805459861u) * 4u;
+    const uint32_t ax[2] = {4u * g[0], 4u * g[0] + 4u}, ay[2] = {g[1] * my, g[1] * my + my}, az[2] = {g[2] * mz, g[2] * mz + mz};
+    float v[8];
+#pragma unroll
+    for (uint32_t c = 0; c < 8; ++c) {
+        const uint32_t x = ax[c & 1u], y = ay[(c >> 1) & 1u], z = az[c >> 2];
+        const uint32_t at = stride ? x + (y + z) : (x ^ (y ^ z)) & (4u * (kHashT - 1u));
+        v[c] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(plane) + at);
+    }
+    float a = 0.0f;
+#pragma unroll
+    for (uint32_t c = 0; c < 8; ++c) {
+        const float w = ((c & 1u) ? f[0] : 1.0f - f[0]) * ((c & 2u) ? f[1] : 1.0f - f[1]) * ((c & 4u) ? f[2] : 1.0f - f[2]);
+        a += w * v[c];
+    }
+    return a;
+}
+
+template <typename T>
+__global__ __launch_bounds__(kPlaneThreads) void forward_planes_kernel(const T* __restrict__ w, uint32_t L,
+                                                                       const rtc8x_radiance_query* __restrict__ in, uint32_t n,
+                                                                       float* __restrict__ out, const float* __restrict__ planes,
+                                                                       uint32_t p_grid, const HashGeom geom, const QueryMask mask)
+{
+    using V = typename Vec8<T>::type;
+    struct Net {
+        T act[kPlaneWaves][64 * kActStride];
+        float pred[kPlaneWaves][64][3];
+    };
+    __shared__ __align__(16) union {
+        float plane[kHashT];
+        Net net;
+    } m;
+    __shared__ uint32_t list[kPlaneTile];
+    __shared__ uint32_t listed;
+    const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
+    const uint32_t r16 = lane & 15, kq = 8 * (lane >> 4);
+    const uint32_t blocks = (n + kPlaneThreads - 1) / kPlaneThreads;
+    uint32_t blk = blockIdx.x;
+    while (blk < blocks) {  // uniform over the workgroup
+        // the next tile of live slots
+        __syncthreads();
+        if (tid == 0) listed = 0;
+        __syncthreads();
+        uint32_t count = 0;
+        while (blk < blocks && count + kPlaneThreads <= kPlaneTile) {
+            const uint32_t s = blk * kPlaneThreads + tid;
+            const bool live = s < n && slot_has_query(mask, s);
+            const uint64_t b = __ballot(live);
+            uint32_t base = 0;
+            if (lane == 0 && b) base = atomicAdd(&listed, (uint32_t)__popcll(b));
+            base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+            if (live) list[base + (uint32_t)__popcll(b & ((1ull << lane) - 1ull))] = s;
+            blk += gridDim.x;
+            __syncthreads();
+            count = listed;
+            __syncthreads();
+        }
+        if (count == 0) continue;
+        // query q of this lane: entry (q * waves + wave) * 64 + lane of the list
+        float p[kPlaneQ][3];
+        u16v feat[kPlaneQ];
+#pragma unroll
+        for (uint32_t q = 0; q < kPlaneQ; ++q) {
+            const uint32_t e = q * kPlaneThreads + tid;
+            query_position01(in[list[min(e, count - 1u)]], p[q]);
+        }
+        for (uint32_t lv = 0; lv < kHashLevels; ++lv) {
+            const uint32_t first = geom.offset[lv] / 2u, entries = level_entries(geom, lv, p_grid);
+            float lo[kPlaneQ];
+#pragma unroll
+            for (uint32_t f = 0; f < 2; ++f) {
+                // memory to LDS directly: the whole plane is in flight at once, without registers
+                const float* src = planes + f * (p_grid / 2u) + first;
+                const uint32_t wave0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid - lane));
+                __syncthreads();
+#pragma unroll 1
+                for (uint32_t k0 = wave0; k0 < entries / 4u; k0 += kPlaneThreads)
+                    if (k0 + lane < entries / 4u)
+                        __builtin_amdgcn_global_load_lds(
+                            (const __attribute__((address_space(1))) void*)(src + 4u * k0 + 4u * lane),
+                            (__attribute__((address_space(3))) void*)(m.plane + 4u * k0), 16, 0, 0);
+                __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's part has landed
+                __syncthreads();
+                const float scale = geom.scale[lv];
+                const uint32_t stride = geom.stride[lv];
+#pragma unroll
+                for (uint32_t q = 0; q < kPlaneQ; ++q) {
+                    if (q * kPlaneThreads < count) {
+                        const float a = plane_sum(m.plane, p[q], scale, stride);
+                        if (f == 0)
+                            lo[q] = a;
+                        else
+                            feat[q][lv] = pack_pair<T>(lo[q], a);
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        // the network, 64 queries at a time (as forward_kernel's inference; the wavefronts are independent)
+        T* A = m.net.act[wave];
+#pragma unroll
+        for (uint32_t q = 0; q < kPlaneQ; ++q) {
+            const uint32_t e = q * kPlaneThreads + tid;
+            if (q * kPlaneThreads + wave * 64u >= count) continue;
+            const uint32_t s = list[min(e, count - 1u)];
+            T* row = &A[lane * kActStride];
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                const uint4 v = make_uint4(feat[q][4 * j], feat[q][4 * j + 1], feat[q][4 * j + 2], feat[q][4 * j + 3]);
+                *reinterpret_cast<uint4*>(&row[8 * j]) = v;
+            }
+            {
+                float t[32];
+                encode_hash_tail(in[s], t);
+#pragma unroll
+                for (int j = 0; j < 32; j += 8) {
+                    V v;
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) v[k] = (T)t[j + k];
+                    *reinterpret_cast<V*>(&row[32 + j]) = v;
+                }
+            }
+            for (uint32_t l = 0; l <= L; ++l) {
+                const bool last = l == L;
+                const T* W = w + (size_t)l * kLayer;
+                const int ntiles = last ? 1 : 4;
+                f4 acc[4][4];
+#pragma unroll
+                for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+                    for (int nt = 0; nt < 4; ++nt) acc[mt][nt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks) {
+                    V a[4];
+#pragma unroll
+                    for (int mt = 0; mt < 4; ++mt)
+                        a[mt] = *reinterpret_cast<const V*>(&A[(mt * 16 + r16) * kActStride + ks * 32 + kq]);
+#pragma unroll
+                    for (int nt = 0; nt < 4; ++nt) {
+                        if (nt < ntiles) {
+                            const V b = *reinterpret_cast<const V*>(&W[(nt * 16 + r16) * kWidth + ks * 32 + kq]);
+#pragma unroll
+                            for (int mt = 0; mt < 4; ++mt) acc[mt][nt] = mfma(b, a[mt], acc[mt][nt]);
+                        }
+                    }
+                }
+                if (!last) {
+#pragma unroll
+                    for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+                        for (int nt = 0; nt < 4; ++nt) {
+                            typename Vec4<T>::type v;
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) v[i] = (T)fmaxf(acc[mt][nt][i], 0.0f);
+                            *reinterpret_cast<typename Vec4<T>::type*>(
+                                &A[(mt * 16 + r16) * kActStride + nt * 16 + 4 * (lane >> 4)]) = v;
+                        }
+                } else if ((lane >> 4) == 0) {
+#pragma unroll
+                    for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+                        for (int i = 0; i < 3; ++i) m.net.pred[wave][mt * 16 + r16][i] = acc[mt][0][i];
+                }
+            }
+            if (e < count) {
+                out[3 * (size_t)s] = m.net.pred[wave][lane][0];
+                out[3 * (size_t)s + 1] = m.net.pred[wave][lane][1];
+                out[3 * (size_t)s + 2] = m.net.pred[wave][lane][2];
+            }
+        }
+    }
+}
+
 // ---------------------------------------------------------------- FP8 inference
 // E4M3 operands on v_mfma_f32_16x16x32_fp8_fp8 with FP32 accumulation.  Weights carry one power-of-two
 // scale per layer (quantize_kernel, from the BF16 EMA weights); activations one power-of-two scale per
@@ -684,11 +904,6 @@ constexpr uint32_t kScatterRange = kHashT / kScatterParts;  // entries per range
 // 16 wavefronts per workgroup instead of 4, or two ranges of a level per workgroup with eight slices
 // (half the atomic instructions per workgroup), both left a 16,384-sample step at 40 us.
 constexpr uint32_t kScatterThreads = 256;
-__device__ __forceinline__ uint32_t level_entries(const HashGeom& gm, uint32_t l, uint32_t p_grid)
-{
-    return ((l + 1 < kHashLevels ? gm.offset[l + 1] : p_grid) - gm.offset[l]) / RTC8X_NRC_HASH_FEATURES;
-}
-
 __global__ __launch_bounds__(kScatterThreads) void grid_scatter_kernel(const rtc8x_radiance_query* __restrict__ in, uint32_t n,
                                                            const float* __restrict__ dE, const HashGeom geom,
                                                            uint32_t p_grid, uint32_t slice_len, float* __restrict__ part)
@@ -926,6 +1141,10 @@ __global__ __launch_bounds__(kReduceThreads) void grad_reduce_kernel(const float
     if (__ballot(nonfinite) != 0 && (threadIdx.x & 63u) == 0) atomicOr(bad, 1u);
 }
 
+// The inference tables are kept twice: as pairs [entry][feature] for gathers from memory, and as planes
+// [feature][entry] for the levels that a workgroup stages in LDS.
+__device__ __forceinline__ uint32_t plane_index(uint32_t j, uint32_t p_grid) { return (j & 1u) * (p_grid / 2u) + (j >> 1); }
+
 struct AdamArgs {
     float lr, beta1, beta2, eps, l2, decay;
     float bc1, bc2;       // 1 - beta^t
@@ -962,8 +1181,8 @@ template <typename T>
 __global__ void adam_kernel(const AdamArgs a, float* __restrict__ master, float* __restrict__ m, float* __restrict__ v,
                             float* __restrict__ ema, const float* __restrict__ grad, uint32_t* __restrict__ bad,
                             T* __restrict__ w, T* __restrict__ wt, T* __restrict__ winf, float* __restrict__ grid_inf,
-                            const float* __restrict__ loss_scale, float* __restrict__ next_scale,
-                            uint32_t* __restrict__ next_bad)
+                            float* __restrict__ grid_planes, const float* __restrict__ loss_scale,
+                            float* __restrict__ next_scale, uint32_t* __restrict__ next_bad)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i == 0) {
@@ -983,7 +1202,10 @@ __global__ void adam_kernel(const AdamArgs a, float* __restrict__ master, float*
     const float e = a.decay * ema[i] + (1.0f - a.decay) * w1;
     ema[i] = e;
     if (i >= a.P_mlp) {  // hash table entry: the FP32 master is the training table
-        grid_inf[i - a.P_mlp] = e / a.ema_bc;
+        const uint32_t j = i - a.P_mlp;
+        const float v = e / a.ema_bc;
+        grid_inf[j] = v;
+        grid_planes[plane_index(j, a.P - a.P_mlp)] = v;
         return;
     }
     w[i] = (T)w1;
@@ -1005,12 +1227,14 @@ __global__ void unscale_kernel(const float* __restrict__ g, uint32_t P, const fl
 
 template <typename T>
 __global__ void convert_kernel(const float* __restrict__ src, uint32_t P, uint32_t L, T* __restrict__ w, T* __restrict__ wt,
-                               T* __restrict__ winf, uint32_t P_total, float* __restrict__ grid_inf)
+                               T* __restrict__ winf, uint32_t P_total, float* __restrict__ grid_inf,
+                               float* __restrict__ grid_planes)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= P_total) return;
     if (i >= P) {
         grid_inf[i - P] = src[i];
+        grid_planes[plane_index(i - P, P_total - P)] = src[i];
         return;
     }
     const T x = (T)src[i];
@@ -1051,6 +1275,7 @@ struct rtc8x_nrc {
     float *master = nullptr, *m = nullptr, *v = nullptr, *ema = nullptr, *grad = nullptr, *gpart = nullptr;
     float* loss_part = nullptr;
     float* grid_inf = nullptr;  // EMA (debiased) hash tables for inference
+    float* grid_planes = nullptr;  // the same, one plane per feature
     float* grid_de = nullptr;   // hash grid: the encoded input's gradient, 32 floats per training sample
     float* grid_part = nullptr; // hash grid: the tables' gradient per slice of the batch (kScatterSlices)
     uint32_t* bad = nullptr;
@@ -1095,12 +1320,37 @@ hipError_t launch_forward_enc(rtc8x_nrc* h, bool train, const void* w, const flo
     return hipGetLastError();
 }
 
+// Inference of n slots by forward_planes_kernel, for 16-bit networks with the hash grid.  A tile of 4,096
+// queries costs a workgroup 66 us for staging the 32 planes, however few queries it holds, and 31 us per 1,024
+// for the gathers and the network; the direct kernel takes 52 us for 131,072 queries, 102 for 262,144 and 797
+// for 2,073,600, this one 75, 94 and 386.  With a mask the number of live slots is not known here: the line lies
+// where a twelfth of them break even.
+template <typename T>
+hipError_t launch_planes(rtc8x_nrc* h, hipStream_t s, const float* in, uint32_t n, float* out, const nrc::QueryMask& mask)
+{
+    int dev = 0, cus = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e != hipSuccess) return e;
+    const uint32_t blocks = (n + nrc::kPlaneThreads - 1) / nrc::kPlaneThreads;
+    hipLaunchKernelGGL((nrc::forward_planes_kernel<T>), dim3(std::min<uint32_t>(blocks, (uint32_t)cus)), dim3(nrc::kPlaneThreads),
+                       0, s, (const T*)h->winf, h->L, (const rtc8x_radiance_query*)in, n, out, (const float*)h->grid_planes,
+                       h->P_grid, h->geom, mask);
+    return hipGetLastError();
+}
+constexpr uint32_t kPlanesMin = 163840, kPlanesMinMasked = 1u << 21;
+
 // train: the working weights and the FP32 master tables; inference: the EMA weights and tables
 template <typename T>
 hipError_t launch_forward(rtc8x_nrc* h, bool train, hipStream_t s, const float* in, uint32_t n, float* out,
                           const float* target, const int32_t* count_dims = nullptr,
                           const nrc::QueryMask& mask = nrc::QueryMask{})
 {
+    if constexpr (sizeof(T) == 2) {
+        if (!train && h->enc == RTC8X_NRC_HASH_GRID && !count_dims && n >= (mask.terms ? kPlanesMinMasked : kPlanesMin))
+            return launch_planes<T>(h, s, in, n, out, mask);
+    }
     const void* w = train ? h->w : h->winf;
     const float* tables = train ? h->master + h->P_mlp : h->grid_inf;
     if (h->enc == RTC8X_NRC_HASH_GRID)
@@ -1142,7 +1392,7 @@ template <typename T>
 hipError_t launch_adam(rtc8x_nrc* h, hipStream_t s, const nrc::AdamArgs& a, uint32_t par)
 {
     hipLaunchKernelGGL((nrc::adam_kernel<T>), dim3((h->P + 255) / 256), dim3(256), 0, s, a, h->master, h->m, h->v, h->ema,
-                       h->grad, h->bad + par, (T*)h->w, (T*)h->wt, (T*)h->winf, h->grid_inf,
+                       h->grad, h->bad + par, (T*)h->w, (T*)h->wt, (T*)h->winf, h->grid_inf, h->grid_planes,
                        (const float*)(h->loss_scale + 2 * par), h->loss_scale + 2 * (par ^ 1u), h->bad + (par ^ 1u));
     return hipGetLastError();
 }
@@ -1151,7 +1401,7 @@ template <typename T>
 hipError_t launch_convert(rtc8x_nrc* h, hipStream_t s)
 {
     hipLaunchKernelGGL((nrc::convert_kernel<T>), dim3((h->P + 255) / 256), dim3(256), 0, s, h->master, h->P_mlp, h->L,
-                       (T*)h->w, (T*)h->wt, (T*)h->winf, h->P, h->grid_inf);
+                       (T*)h->w, (T*)h->wt, (T*)h->winf, h->P, h->grid_inf, h->grid_planes);
     return hipGetLastError();
 }
 
@@ -1222,7 +1472,7 @@ extern "C" rtc8x_status rtc8x_nrc_destroy(rtc8x_nrc* h)
 try {
     if (!h) return RTC8X_OK;
     void* ptrs[] = {h->master, h->m, h->v, h->ema, h->grad, h->gpart, h->loss_part, h->bad, h->w, h->wt, h->winf, h->hbuf, h->dout,
-                    h->grid_inf, h->grid_de, h->grid_part, h->w8, h->w8_inv, h->loss_scale};
+                    h->grid_inf, h->grid_planes, h->grid_de, h->grid_part, h->w8, h->w8_inv, h->loss_scale};
     for (void* p : ptrs)
         if (p) RTC8X_HIP(hipFree(p));
     delete h;
@@ -1265,6 +1515,7 @@ try {
               alloc((void**)&h->gpart, 4 * P_mlp * max_blocks) && alloc((void**)&h->loss_part, 4 * max_waves) &&
               alloc((void**)&h->bad, 8) && alloc((void**)&h->loss_scale, 16) && alloc(&h->w, h->tsize * P_mlp) && alloc(&h->wt, h->tsize * h->PT) &&
               alloc(&h->winf, h->tsize * P_mlp) && (h->P_grid == 0 || alloc((void**)&h->grid_inf, 4 * (size_t)h->P_grid)) &&
+              (h->P_grid == 0 || alloc((void**)&h->grid_planes, 4 * (size_t)h->P_grid)) &&
               (h->P_grid == 0 || alloc((void**)&h->grid_de, 4 * 32 * (size_t)nrc::kMaxTrain)) &&
               (h->P_grid == 0 || alloc((void**)&h->grid_part, 4 * (size_t)h->P_grid * nrc::kScatterSlices)) &&
               alloc(&h->hbuf, h->tsize * 64 * (size_t)(h->L + 1) * nrc::kMaxTrain) &&
