@@ -807,10 +807,16 @@ __global__ __launch_bounds__(256) void quantize_kernel(const __bf16* __restrict_
 // Inference with E4M3 operands: the BF16 forward's structure (encoding into the LDS tile, then per
 // layer 4 x 4 x 2 MFMAs per wavefront), with each layer's activations scaled and quantised on the way
 // from LDS into the A operands.
-template <int ENC>
+//
+// OWN: the workgroup quantises the BF16 weights itself, into LDS (quantize_kernel's scales and bytes; a
+// wavefront takes every fourth layer), and w8 and w_inv are not read.
+constexpr uint32_t kOwnRow = 72;  // bytes of a quantised weight row in LDS (64, and 8 against bank conflicts)
+__host__ __device__ constexpr uint32_t own_bytes(uint32_t L) { return (L * kWidth + kOutPad) * kOwnRow; }
+template <int ENC, bool OWN>
 // (256, 3) as for forward_kernel: four waves per SIMD instead of two (0.20 ms per 2^21 queries at L = 5,
 // against 0.29 ms)
-__global__ __launch_bounds__(256, 3) void forward_fp8_kernel(const uint8_t* __restrict__ w8, const float* __restrict__ w_inv,
+__global__ __launch_bounds__(256, 3) void forward_fp8_kernel(const __bf16* __restrict__ winf, const uint8_t* __restrict__ w8,
+                                                          const float* __restrict__ w_inv,
                                                           uint32_t L, const rtc8x_radiance_query* __restrict__ in,
                                                           uint32_t n, float* __restrict__ out,
                                                           const float* __restrict__ tables, const HashGeom geom,
@@ -827,6 +833,39 @@ __global__ __launch_bounds__(256, 3) void forward_fp8_kernel(const uint8_t* __re
     // as in forward_kernel: slots without a query are skipped (their zero rows also leave the tile's
     // activation scales to the queries)
     const bool live = s < n && slot_has_query(mask, s);
+    extern __shared__ __align__(16) uint8_t own[];
+    __shared__ float own_inv[kMaxLayers + 1];
+    if constexpr (OWN) {
+        if (!__syncthreads_or(live)) return;
+        for (uint32_t l = wave; l <= L; l += 4) {
+            // chunks of eight weights; a hidden layer has eight per lane, the output layer two
+            constexpr uint32_t kChunks = kLayer / 8 / 64;
+            const uint32_t chunks = l < L ? kChunks : kOutPad * kWidth / 8 / 64;
+            V v[kChunks];
+            float m = 0.0f;
+#pragma unroll
+            for (uint32_t j = 0; j < kChunks; ++j)
+                if (j < chunks) v[j] = *reinterpret_cast<const V*>(winf + (size_t)l * kLayer + 8 * (64 * j + lane));
+#pragma unroll
+            for (uint32_t j = 0; j < kChunks; ++j)
+                if (j < chunks) {
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) m = fmaxf(m, fabsf((float)v[j][k]));
+                }
+            for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+            const float sc = pow2_scale(m);
+            if (lane == 0) own_inv[l] = 1.0f / sc;
+#pragma unroll
+            for (uint32_t j = 0; j < kChunks; ++j)
+                if (j < chunks) {
+                    float x[8];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) x[k] = (float)v[j][k] * sc;
+                    *reinterpret_cast<long*>(&own[(l * kWidth + 8 * j + lane / 8) * kOwnRow + 8 * (lane % 8)]) = pack_fp8(x);
+                }
+        }
+        __syncthreads();
+    }
     if (__ballot(live) == 0) return;
     T* A = act[wave];
     if constexpr (ENC == kEncHash) {
@@ -855,7 +894,8 @@ __global__ __launch_bounds__(256, 3) void forward_fp8_kernel(const uint8_t* __re
     float sa = 1.0f;
     for (uint32_t l = 0; l <= L; ++l) {
         const bool last = l == L;
-        const uint8_t* W = w8 + (size_t)l * kLayer;
+        const uint8_t* W = OWN ? &own[l * kWidth * kOwnRow] : w8 + (size_t)l * kLayer;
+        constexpr uint32_t kRowW = OWN ? kOwnRow : kWidth;
         const int ntiles = last ? 1 : 4;
         long a[2][4];
         if (l == 0) {
@@ -886,7 +926,7 @@ __global__ __launch_bounds__(256, 3) void forward_fp8_kernel(const uint8_t* __re
                 for (int mt = 0; mt < 4; ++mt)
                     __builtin_memcpy(&a[ks][mt], &A8[(mt * 16 + r16) * kRow8 + ks * 32 + kq], sizeof(long));
         }
-        const float unscale = w_inv[l] / sa;
+        const float unscale = (OWN ? own_inv[l] : w_inv[l]) / sa;
         // Weights as the A operand, activations as B: the product is the layer's output transposed, so
         // acc[mt][nt][i] is feature nt*16 + 4*(lane>>4) + i of query mt*16 + (lane&15).
         f4 acc[4][4];
@@ -899,7 +939,7 @@ __global__ __launch_bounds__(256, 3) void forward_fp8_kernel(const uint8_t* __re
 #pragma unroll
             for (int nt = 0; nt < 4; ++nt) {
                 if (nt < ntiles) {
-                    const long b = *reinterpret_cast<const long*>(&W[(nt * 16 + r16) * kWidth + ks * 32 + kq]);
+                    const long b = *reinterpret_cast<const long*>(&W[(nt * 16 + r16) * kRowW + ks * 32 + kq]);
 #pragma unroll
                     for (int mt = 0; mt < 4; ++mt)
                         acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(b, a[ks][mt], acc[mt][nt], 0, 0, 0);
@@ -1476,20 +1516,38 @@ hipError_t with_type(const rtc8x_nrc* h, F&& f)
 #define RTC8X_WITH_TYPE(h, call) with_type(h, [&](auto tag) { using T = std::remove_pointer_t<decltype(tag)>; return call; })
 bool is_fp8(const rtc8x_nrc* h) { return h->desc.precision == RTC8X_NRC_BF16_FP8; }
 
+// The forward kernel quantises the weights itself in launches of up to kOwnBlocks workgroups, where the launch
+// of quantize_kernel costs 6 to 9 us and the quantising 1 (62,793 queries, L = 2: hash 33.5 us with the launch, 27.0
+// without; triangle wave 14.6 and 9.1), and in the hash grid's larger ones, where weights in LDS leave the L1 to the
+// gathers (2^21 queries: 700 us and 649; L = 5 706 and 628).  A larger triangle-wave launch is bound by what each
+// workgroup repeats and by occupancy (2^21 queries: 108 us with quantize_kernel, 131 without; L = 5 184 and 262; at
+// 150,000 still 27.8 and 30.6); in a larger masked one each workgroup may hold few queries.
+constexpr uint32_t kOwnBlocks = 512;
+
+template <int ENC>
+void launch_fp8(rtc8x_nrc* h, hipStream_t s, const float* in, uint32_t n, float* out, const int32_t* count_dims,
+                const nrc::QueryMask& mask)
+{
+    const uint32_t blocks = (n + 255) / 256;
+    const auto* w = (const __bf16*)h->winf;
+    const auto* q = (const rtc8x_radiance_query*)in;
+    if (blocks <= kOwnBlocks || (ENC == RTC8X_NRC_HASH_GRID && !mask.terms)) {
+        hipLaunchKernelGGL((nrc::forward_fp8_kernel<ENC, true>), dim3(blocks), dim3(256), nrc::own_bytes(h->L), s, w, h->w8,
+                           h->w8_inv, h->L, q, n, out, h->grid_inf, h->geom, count_dims, mask);
+        return;
+    }
+    hipLaunchKernelGGL(nrc::quantize_kernel, dim3(h->L + 1), dim3(256), 0, s, w, h->L, h->w8, h->w8_inv);
+    hipLaunchKernelGGL((nrc::forward_fp8_kernel<ENC, false>), dim3(blocks), dim3(256), 0, s, w, h->w8, h->w8_inv, h->L, q, n,
+                       out, h->grid_inf, h->geom, count_dims, mask);
+}
+
 hipError_t launch_forward_fp8(rtc8x_nrc* h, hipStream_t s, const float* in, uint32_t n, float* out,
                               const int32_t* count_dims = nullptr, const nrc::QueryMask& mask = nrc::QueryMask{})
 {
-    hipLaunchKernelGGL(nrc::quantize_kernel, dim3(h->L + 1), dim3(256), 0, s, (const __bf16*)h->winf, h->L, h->w8,
-                       h->w8_inv);
-    const uint32_t blocks = (n + 255) / 256;
     if (h->enc == RTC8X_NRC_HASH_GRID)
-        hipLaunchKernelGGL((nrc::forward_fp8_kernel<RTC8X_NRC_HASH_GRID>), dim3(blocks), dim3(256), 0, s, h->w8,
-                           h->w8_inv, h->L, (const rtc8x_radiance_query*)in, n, out, h->grid_inf, h->geom, count_dims,
-                           mask);
+        launch_fp8<RTC8X_NRC_HASH_GRID>(h, s, in, n, out, count_dims, mask);
     else
-        hipLaunchKernelGGL((nrc::forward_fp8_kernel<RTC8X_NRC_TRIANGLE_WAVE>), dim3(blocks), dim3(256), 0, s, h->w8,
-                           h->w8_inv, h->L, (const rtc8x_radiance_query*)in, n, out, h->grid_inf, h->geom, count_dims,
-                           mask);
+        launch_fp8<RTC8X_NRC_TRIANGLE_WAVE>(h, s, in, n, out, count_dims, mask);
     return hipGetLastError();
 }
 
