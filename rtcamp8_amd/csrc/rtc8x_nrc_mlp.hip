@@ -1196,13 +1196,17 @@ __global__ __launch_bounds__(64 * WPB) void backward_kernel(const T* __restrict_
 // c, c + 16, c + 32, ... (four loads in flight), and the 16 slices are added in a fixed order, so the
 // result does not depend on scheduling.  The other workgroups sum 1,024 hash-table gradients each over
 // the scatter's slices (entries P .. P_total; none without the hash grid).  Any non-finite sum sets *bad.
+// A gradient that is handed out (rtc8x_nrc_gradient) is divided by the loss scale here and sets no flag
+// (bad NULL): a launch for the division and a clearing of the flag behind it were 9 of a 16,384-sample
+// gradient's 78 us.
 constexpr uint32_t kReduceSlices = 16;
 constexpr uint32_t kReduceThreads = 64 * kReduceSlices;
 __global__ __launch_bounds__(kReduceThreads) void grad_reduce_kernel(const float* __restrict__ gpart, uint32_t nblocks, uint32_t P,
                                                           uint32_t P_total, const float* __restrict__ grid_part,
                                                           uint32_t slices, float* __restrict__ grad,
-                                                          uint32_t* __restrict__ bad)
+                                                          uint32_t* __restrict__ bad, const float* __restrict__ loss_scale)
 {
+    const float scale = bad ? 1.0f : *loss_scale;
     const uint32_t mlp_groups = (P + 63) / 64;
     bool nonfinite = false;
     if (blockIdx.x < mlp_groups) {
@@ -1223,7 +1227,7 @@ __global__ __launch_bounds__(kReduceThreads) void grad_reduce_kernel(const float
             float g = part[0][il];
 #pragma unroll
             for (uint32_t k = 1; k < kReduceSlices; ++k) g += part[k][il];
-            grad[i] = g;
+            grad[i] = bad ? g : g / scale;
             nonfinite = !isfinite(g);
         }
     } else {
@@ -1231,11 +1235,11 @@ __global__ __launch_bounds__(kReduceThreads) void grad_reduce_kernel(const float
         if (j < p_grid) {
             float sum = grid_part[j];
             for (uint32_t h = 1; h < slices; ++h) sum += grid_part[h * p_grid + j];
-            grad[P + j] = sum;
+            grad[P + j] = bad ? sum : sum / scale;
             nonfinite = !isfinite(sum);
         }
     }
-    if (__ballot(nonfinite) != 0 && (threadIdx.x & 63u) == 0) atomicOr(bad, 1u);
+    if (bad && __ballot(nonfinite) != 0 && (threadIdx.x & 63u) == 0) atomicOr(bad, 1u);
 }
 
 // The inference tables are kept twice: as pairs [entry][feature] for gathers from memory, and as planes
@@ -1312,14 +1316,6 @@ __global__ void adam_kernel(const AdamArgs a, float* __restrict__ master, float*
         wt[(size_t)l * kLayer + in * kWidth + out] = (T)w1;
     else
         wt[(size_t)a.L * kLayer + in * kOutT + out] = (T)w1;
-}
-
-// g / loss scale, for the gradient handed out by rtc8x_nrc_gradient
-__global__ void unscale_kernel(const float* __restrict__ g, uint32_t P, const float* __restrict__ state,
-                               float* __restrict__ out)
-{
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < P) out[i] = g[i] / state[0];
 }
 
 template <typename T>
@@ -1567,16 +1563,17 @@ rtc8x_status reset_from_master(rtc8x_nrc* h)
     return RTC8X_OK;
 }
 
-// forward (train) + backward + ordered reduction into h->grad; returns the loss sum in *loss_sum when set
-rtc8x_status gradient_pass(rtc8x_nrc* h, hipStream_t s, const float* in, const float* target, uint32_t n)
+// forward (train) + backward + ordered reduction into h->grad, or, divided by the loss scale, into grad_out
+rtc8x_status gradient_pass(rtc8x_nrc* h, hipStream_t s, const float* in, const float* target, uint32_t n,
+                           float* grad_out = nullptr)
 {
     RTC8X_HIP(RTC8X_WITH_TYPE(h, launch_forward<T>(h, true, s, in, n, nullptr, target)));
     RTC8X_HIP(RTC8X_WITH_TYPE(h, launch_backward<T>(h, s, in, n)));
     // the step's flag is zero here: set so at creation, cleared by the previous step's optimiser kernel
-    // (and after a gradient handed out by rtc8x_nrc_gradient)
     const uint32_t groups = (h->P_mlp + 63) / 64 + (h->P - h->P_mlp + nrc::kReduceThreads - 1) / nrc::kReduceThreads;
     hipLaunchKernelGGL(nrc::grad_reduce_kernel, dim3(groups), dim3(nrc::kReduceThreads), 0, s, h->gpart, train_blocks(n), h->P_mlp, h->P,
-                       (const float*)h->grid_part, scatter_slices(n), h->grad, h->bad + (h->step & 1u));
+                       (const float*)h->grid_part, scatter_slices(n), grad_out ? grad_out : h->grad,
+                       grad_out ? nullptr : h->bad + (h->step & 1u), scale_state(h));
     RTC8X_HIP(hipGetLastError());
     return RTC8X_OK;
 }
@@ -1770,13 +1767,7 @@ try {
     RTC8X_REQUIRE(h && in && target && grad, "rtc8x_nrc_gradient: NULL argument");
     RTC8X_REQUIRE(n > 0 && n <= nrc::kMaxTrain, "rtc8x_nrc_gradient: n must be in [1, %u]", nrc::kMaxTrain);
     hipStream_t s = (hipStream_t)stream;
-    rtc8x_status st = gradient_pass(h, s, in, target, n);
-    if (st != RTC8X_OK) return st;
-    hipLaunchKernelGGL(nrc::unscale_kernel, dim3((h->P + 255) / 256), dim3(256), 0, s, (const float*)h->grad, h->P,
-                       scale_state(h), grad);
-    RTC8X_HIP(hipGetLastError());
-    RTC8X_HIP(hipMemsetAsync(h->bad + (h->step & 1u), 0, sizeof(uint32_t), s));
-    return RTC8X_OK;
+    return gradient_pass(h, s, in, target, n, grad);
 }
 RTC8X_CATCH_ALL("rtc8x_nrc_gradient")
 
