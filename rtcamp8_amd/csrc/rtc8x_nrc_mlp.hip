@@ -1001,6 +1001,57 @@ constexpr uint32_t kScatterRange = kHashT / kScatterParts;  // entries per range
 // 16 wavefronts per workgroup instead of 4, or two ranges of a level per workgroup with eight slices
 // (half the atomic instructions per workgroup), both left a 16,384-sample step at 40 us.
 constexpr uint32_t kScatterThreads = 256;
+// The contributions of samples s0 .. s1 to the range r of level lv (DENSE: the entries e with
+// e % kScatterParts == r, otherwise those from r * kScatterRange on).  The two kinds are compiled apart: chosen
+// per corner, the choice took two scalar branches for each of a sample's eight (a 16,384-sample step: 30.4 us;
+// apart, and with the gradients level by level, 29.4).
+template <bool DENSE>
+__device__ __forceinline__ void scatter_slice(const rtc8x_radiance_query* __restrict__ in, const float* __restrict__ dE,
+                                              const HashGeom& geom, uint32_t n, uint32_t lv, uint32_t r, uint32_t s0,
+                                              uint32_t s1, float* acc)
+{
+    constexpr uint32_t kBatch = 4;  // samples per lane whose loads are issued together
+    const float scale = geom.scale[lv];
+    const uint32_t my = DENSE ? geom.stride[lv] : 2654435761u, mz = DENSE ? geom.stride[lv] * geom.stride[lv] : 805459861u;
+    for (uint32_t sb = s0 + threadIdx.x; sb < s1; sb += kBatch * kScatterThreads) {
+        float p[kBatch][3];
+        float2 g[kBatch];
+#pragma unroll
+        for (uint32_t k = 0; k < kBatch; ++k) {
+            const uint32_t sm = min(sb + k * kScatterThreads, s1 - 1);
+            query_position01(in[sm], p[k]);
+            g[k] = reinterpret_cast<const float2*>(dE)[(size_t)lv * n + sm];
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kBatch; ++k) {
+            if (sb + k * kScatterThreads < s1) {
+                uint32_t gi[3];
+                float f[3];
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    const float pos = p[k][d] * scale + 0.5f;
+                    const float fl = floorf(pos);
+                    f[d] = pos - fl;
+                    gi[d] = (uint32_t)fl;
+                }
+                const uint32_t y[2] = {gi[1] * my, gi[1] * my + my}, z[2] = {gi[2] * mz, gi[2] * mz + mz};
+#pragma unroll
+                for (uint32_t c = 0; c < 8; ++c) {
+                    const uint32_t x = gi[0] + (c & 1u), cy = y[(c >> 1) & 1u], cz = z[c >> 2];
+                    const float w = ((c & 1u) ? f[0] : 1.0f - f[0]) * ((c & 2u) ? f[1] : 1.0f - f[1]) * ((c & 4u) ? f[2] : 1.0f - f[2]);
+                    const uint32_t e = DENSE ? x + cy + cz : (x ^ cy ^ cz) & (kHashT - 1u);
+                    const uint32_t part = DENSE ? e % kScatterParts : e / kScatterRange;
+                    const uint32_t j = DENSE ? e / kScatterParts : e % kScatterRange;
+                    if (part == r) {
+                        atomicAdd(&acc[2 * j], w * g[k].x);
+                        atomicAdd(&acc[2 * j + 1], w * g[k].y);
+                    }
+                }
+            }
+        }
+    }
+}
+
 __global__ __launch_bounds__(kScatterThreads) void grid_scatter_kernel(const rtc8x_radiance_query* __restrict__ in, uint32_t n,
                                                            const float* __restrict__ dE, const HashGeom geom,
                                                            uint32_t p_grid, uint32_t slice_len, float* __restrict__ part)
@@ -1020,39 +1071,11 @@ __global__ __launch_bounds__(kScatterThreads) void grid_scatter_kernel(const rtc
     float2* acc2 = reinterpret_cast<float2*>(acc);
     for (uint32_t i = threadIdx.x; i < owned; i += kScatterThreads) acc2[i] = float2{0.0f, 0.0f};
     __syncthreads();
-    const uint32_t s1 = min(n, (slice + 1) * slice_len);
-    constexpr uint32_t kBatch = 4;  // samples per lane whose loads are issued together
-    for (uint32_t sb = slice * slice_len + threadIdx.x; sb < s1; sb += kBatch * kScatterThreads) {
-        float p[kBatch][3];
-        float2 g[kBatch];
-#pragma unroll
-        for (uint32_t k = 0; k < kBatch; ++k) {
-            const uint32_t sm = min(sb + k * kScatterThreads, s1 - 1);
-            query_position01(in[sm], p[k]);
-            __builtin_memcpy(&g[k], dE + (size_t)sm * 32 + 2 * lv, sizeof(float2));
-        }
-#pragma unroll
-        for (uint32_t k = 0; k < kBatch; ++k) {
-            if (sb + k * kScatterThreads < s1) {
-                uint32_t gi[3];
-                float f[3];
-                hash_cell(geom, lv, p[k], gi, f);
-#pragma unroll
-                for (uint32_t c = 0; c < 8; ++c) {
-                    uint32_t idx;
-                    float w;
-                    hash_corner(geom, lv, gi, f, c, idx, w);
-                    const uint32_t e = (idx - geom.offset[lv]) / 2u;
-                    const bool mine = dense ? e % kScatterParts == r : e >= e0 && e < e1;
-                    const uint32_t j = dense ? e / kScatterParts : e - e0;
-                    if (mine) {
-                        atomicAdd(&acc[2 * j], w * g[k].x);
-                        atomicAdd(&acc[2 * j + 1], w * g[k].y);
-                    }
-                }
-            }
-        }
-    }
+    const uint32_t s0 = slice * slice_len, s1 = min(n, s0 + slice_len);
+    if (dense)
+        scatter_slice<true>(in, dE, geom, n, lv, r, s0, s1, acc);
+    else
+        scatter_slice<false>(in, dE, geom, n, lv, r, s0, s1, acc);
     __syncthreads();
     float2* out = reinterpret_cast<float2*>(part + (size_t)slice * p_grid + geom.offset[lv]);
     for (uint32_t i = threadIdx.x; i < owned; i += kScatterThreads) out[dense ? i * kScatterParts + r : e0 + i] = acc2[i];
@@ -1071,6 +1094,7 @@ __global__ __launch_bounds__(64 * WPB) void backward_kernel(const T* __restrict_
     __shared__ __align__(16) T dzs[kSampleMajor ? SB * kActStride : 8];   // dZ, sample-major [sample][out]
     __shared__ __align__(16) T dzf[64 * CS];                              // dZ, feature-major [out][sample]
     __shared__ __align__(16) T hf[64 * CS];     // layer input H, feature-major [in][sample]
+    static_assert(sizeof(hf) >= SB * 33 * sizeof(float), "holds the encoded input's gradient");
     const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const uint32_t r16 = lane & 15, kq = 8 * (lane >> 4);
     const uint32_t b0 = blockIdx.x * SB;
@@ -1155,7 +1179,7 @@ __global__ __launch_bounds__(64 * WPB) void backward_kernel(const T* __restrict_
         }
         __syncthreads();
         if (ENC == kEncHash && l == 0) {
-            // dE for the 32 grid features, FP32, sample-major in the (now free) H tile
+            // dE for the 32 grid features, FP32, sample-major in the (now free) H tile (33 floats per row)
             float* dE = reinterpret_cast<float*>(hf);
 #pragma unroll
             for (int mt = 0; mt < 4; ++mt)
@@ -1163,14 +1187,13 @@ __global__ __launch_bounds__(64 * WPB) void backward_kernel(const T* __restrict_
                 for (int nt = 0; nt < 2; ++nt)
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
-                        dE[(wave * 64 + mt * 16 + 4 * (lane >> 4) + i) * 32 + nt * 16 + r16] = acc[mt][nt][i];
+                        dE[(wave * 64 + mt * 16 + 4 * (lane >> 4) + i) * 33 + nt * 16 + r16] = acc[mt][nt][i];
             __syncthreads();
-            // the rows of dE go out for grid_scatter_kernel, 16 bytes per lane and store
-            for (uint32_t i = tid; i < SB * 8; i += SB) {
-                const uint32_t sm = i >> 3;
-                if (b0 + sm < n)
-                    *reinterpret_cast<f4*>(dEout + (size_t)(b0 + sm) * 32 + 4 * (i & 7u)) =
-                        *reinterpret_cast<const f4*>(dE + sm * 32 + 4 * (i & 7u));
+            // out for grid_scatter_kernel, level by level
+            if (b0 + tid < n) {
+#pragma unroll
+                for (uint32_t lv = 0; lv < kHashLevels; ++lv)
+                    reinterpret_cast<float2*>(dEout)[(size_t)lv * n + b0 + tid] = float2{dE[tid * 33 + 2 * lv], dE[tid * 33 + 2 * lv + 1]};
             }
             break;
         }
@@ -1197,7 +1220,7 @@ __global__ __launch_bounds__(64 * WPB) void backward_kernel(const T* __restrict_
 // result does not depend on scheduling.  The other workgroups sum 1,024 hash-table gradients each over
 // the scatter's slices (entries P .. P_total; none without the hash grid).  Any non-finite sum sets *bad.
 // A gradient that is handed out (rtc8x_nrc_gradient) is divided by the loss scale here and sets no flag
-// (bad NULL): a launch for the division and a clearing of the flag behind it were 9 of a 16,384-sample
+// (bad NULL): a launch for the division and a clearing of the flag behind it were 5 of a 16,384-sample
 // gradient's 78 us.
 constexpr uint32_t kReduceSlices = 16;
 constexpr uint32_t kReduceThreads = 64 * kReduceSlices;
@@ -1369,7 +1392,7 @@ struct rtc8x_nrc {
     float* loss_part = nullptr;
     float* grid_inf = nullptr;  // EMA (debiased) hash tables for inference
     float* grid_planes = nullptr;  // the same, one plane per feature
-    float* grid_de = nullptr;   // hash grid: the encoded input's gradient, 32 floats per training sample
+    float* grid_de = nullptr;   // hash grid: the encoded input's gradient, a feature pair per level and training sample
     float* grid_part = nullptr; // hash grid: the tables' gradient per slice of the batch (kScatterSlices)
     uint32_t* bad = nullptr;
     float* loss_scale = nullptr;  // two [scale, finite steps since it changed] states, by step parity
