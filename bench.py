@@ -597,7 +597,7 @@ def global_majorant_leg(scene, pt, spp: int, steps: int, stream) -> dict:
            "path_vertices_per_s": c["vertices"] / wall, "paths_per_s": c["paths"] / wall,
            "vertices_per_path": c["vertices"] / max(c["paths"], 1), "lookups_per_path": c["lookups"] / max(c["paths"], 1),
            "hbm_roofline_frac": lookups_per_launch * BYTES_PER_LOOKUP / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
-           "kernel": "wavefront_kernel<PATH_TRACE, GLOBAL_MAJORANT>"}
+           "kernel": "slots_kernel<PATH_TRACE, GLOBAL_MAJORANT>"}
     out["latency_roofline"] = latency_roofline(scene, params, lookups_per_launch, out["lookups_per_path"],
                                                c["lookups"] / sum(kernel_ms) * 1e3, out["paths_per_s"])
     pt.stats.fill(0)
@@ -710,8 +710,8 @@ def main() -> int:
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": achieved_gbs / HBM_PEAK_GBS,
-            "traffic": traffic_from_profiles(f"wavefront_kernel_{args.tracking}", cfg.name),
-            "kernel": f"wavefront_kernel<PATH_TRACE, {args.tracking.upper()}_MAJORANT>",
+            "traffic": traffic_from_profiles(f"slots_kernel_{args.tracking}", cfg.name),
+            "kernel": f"slots_kernel<PATH_TRACE, {args.tracking.upper()}_MAJORANT>",
             "kernel_ms_avg": float(np.mean(kernel_ms)),
             "algorithmic_bytes_per_launch": lookups_per_launch * BYTES_PER_LOOKUP,
         },
