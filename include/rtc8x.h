@@ -168,7 +168,7 @@ typedef struct rtc8x_grid {
      * a leaf (8 words) or per table entry of a lower (64 words) / upper (512 words) node, bit n of word
      * n / 64 for offset n.  A set bit on an internal table entry marks an active tile.  Decoded grids
      * carry them; the encoder writes them back, and treats NULL as every leaf voxel active and every
-     * tile inactive.  Never uploaded: in a device grid the library keeps its lookup bricks here (opaque). */
+     * tile inactive.  Never uploaded. */
     const uint64_t* leaf_masks;          /* num_leaves x 8 */
     const uint64_t* lower_masks;         /* num_lower x 64 */
     const uint64_t* upper_masks;         /* num_upper x 512 */
@@ -194,6 +194,15 @@ typedef struct rtc8x_grid {
     uint32_t region_cells;
     float region_unit;
     const uint8_t* region_majorants;
+    /* Lookup bricks (library-built with the leaf map, optional): copies of the voxels laid out by trilinear
+     * stencil, 9,216 bytes per 8^3 block that is not inside one tile, and one u32 per block of the leaf map;
+     * about 4.5 times the bytes of leaf_values.  A cache of the tables: lookups without them give the same
+     * values.  The layout is the library's own.  brick_key names the tables they were filled from; a grid
+     * with other leaf_values, tile_values or leaf_map is looked up without them.  Values changed in place need
+     * new bricks. */
+    const float* bricks;
+    const uint32_t* brick_map;
+    uint64_t brick_key;
 } rtc8x_grid;
 
 #define RTC8X_MAX_REGIONS 32768

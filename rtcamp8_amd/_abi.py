@@ -75,6 +75,9 @@ class Grid(C.Structure):
         ("region_cells", C.c_uint32),
         ("region_unit", C.c_float),
         ("region_majorants", C.c_void_p),
+        ("bricks", C.c_void_p),
+        ("brick_map", C.c_void_p),
+        ("brick_key", C.c_uint64),
     ]
 
 

@@ -187,9 +187,9 @@ __device__ __forceinline__ V3 world_to_index(const rtc8x_grid& g, float px, floa
 // lower corner is the 32 bytes of its quad and the next, in one block whatever faces it crosses: one map
 // load, then two 16-byte loads, with no branch in between.  brick_map[block] is the brick's first quad.  A
 // block that is the same tile as its seven upper neighbours names the two quads of that tile's value
-// instead, with kSharedBrick set: one address for all lanes in empty space.  Device grids carry the two
-// pointers in the host-only mask fields (lower_masks: the bricks, leaf_masks: the map), valid when
-// upper_masks is their tag.
+// instead, with kSharedBrick set: one address for all lanes in empty space.  The bricks hold copies of the
+// values, so a grid uses them only while its tables are the ones they were filled from (brick_key): a caller
+// that puts other tables into a copy of a device grid gets lookups of those.
 //
 // The trackers' lookups are random reads, and the rate of cache lines that miss the L2 bounds them: about
 // 56 G lines/s, whether the lines lie in 64 or in 512 MB.  A stencil in the leaves' own layout touches 2.8
@@ -200,16 +200,12 @@ __device__ __forceinline__ V3 world_to_index(const rtc8x_grid& g, float px, floa
 // ones, the dense 128^3 cloud's 256 x 256 frame of 4 samples from 1.37 to 1.19 ms.
 constexpr uint32_t kBrickQuads = 8 * 8 * 9;
 constexpr uint32_t kSharedBrick = 0x80000000u;
-constexpr uint64_t kBrickTag = 0x6272636b38783921ull;
-__host__ __device__ __forceinline__ uint64_t brick_tag(const void* values, const void* map)
+__host__ __device__ __forceinline__ uint64_t brick_key(const rtc8x_grid& g)
 {
-    return (uint64_t)(uintptr_t)values ^ (uint64_t)(uintptr_t)map ^ kBrickTag;
+    return (uint64_t)(uintptr_t)g.bricks ^ (uint64_t)(uintptr_t)g.brick_map << 1 ^ (uint64_t)(uintptr_t)g.leaf_map << 2 ^
+           (uint64_t)(uintptr_t)g.leaf_values << 3 ^ (uint64_t)(uintptr_t)g.tile_values << 4;
 }
-__host__ __device__ __forceinline__ bool brick_tagged(const rtc8x_grid& g)
-{
-    return g.lower_masks && (uint64_t)(uintptr_t)g.upper_masks == brick_tag(g.lower_masks, g.leaf_masks);
-}
-__host__ __device__ __forceinline__ bool has_bricks(const rtc8x_grid& g) { return g.leaf_map && brick_tagged(g); }
+__host__ __device__ __forceinline__ bool has_bricks(const rtc8x_grid& g) { return g.bricks && g.brick_key == brick_key(g); }
 
 // One lookup through the tree (or the leaf map), tap by tap: positions outside the bricks, and grids
 // without them.  The x planes are looped over to keep the code small.
@@ -236,15 +232,14 @@ __device__ __forceinline__ float trilinear_tree(const rtc8x_grid& g, V3 idx)
 }
 
 // SampleFromVoxels<Acc,1,false>::operator() (util/SampleFromVoxels.h:419-460) with Floor (:58-65), for
-// S index-space positions at once.  All loads are issued in two rounds (every position's brick, then every
+// S index-space positions at once; have: has_bricks(g).  All loads are issued in two rounds (every position's brick, then every
 // position's voxels), so the lookups of a batch overlap instead of each waiting on the one before.  The
 // lerps are the reference's, in its order.
 template <uint32_t S>
-__device__ __forceinline__ void trilinear_batch(const rtc8x_grid& g, const V3 (&idx)[S], float (&out)[S])
+__device__ __forceinline__ void trilinear_batch(const rtc8x_grid& g, bool have, const V3 (&idx)[S], float (&out)[S])
 {
-    const bool have = has_bricks(g);  // uniform
-    const float4* const bricks = reinterpret_cast<const float4*>(g.lower_masks);
-    const uint32_t* const map = reinterpret_cast<const uint32_t*>(g.leaf_masks);
+    const float4* const bricks = reinterpret_cast<const float4*>(g.bricks);
+    const uint32_t* const map = g.brick_map;
     const uint32_t d0 = (uint32_t)g.leaf_map_dims[0], d1 = (uint32_t)g.leaf_map_dims[1], d2 = (uint32_t)g.leaf_map_dims[2];
     bool in[S];
     if (have) {
@@ -294,11 +289,11 @@ __device__ __forceinline__ void trilinear_batch(const rtc8x_grid& g, const V3 (&
         if (!in[s]) out[s] = trilinear_tree(g, idx[s]);
 }
 
-__device__ __forceinline__ float trilinear(const rtc8x_grid& g, V3 idx)
+__device__ __forceinline__ float trilinear(const rtc8x_grid& g, bool have, V3 idx)
 {
     const V3 in[1] = {idx};
     float out[1];
-    trilinear_batch<1>(g, in, out);
+    trilinear_batch<1>(g, have, in, out);
     return out[0];
 }
 
@@ -306,9 +301,11 @@ struct Medium {
     float coeff;
     float majorant;
     uint32_t lookups;
+    bool bricks;  // has_bricks of the grid (uniform)
     bool normal;  // every majorant lies in div_normal's range (uniform)
-    __device__ __forceinline__ void init(const rtc8x_grid& g, float density_coeff)
+    __device__ __forceinline__ void init(const rtc8x_grid& g, float density_coeff, bool have_bricks)
     {
+        bricks = have_bricks;
         coeff = density_coeff;
         majorant = density_coeff * g.max_value;
         lookups = 0;
@@ -321,30 +318,30 @@ struct Medium {
 };
 
 // Density coefficient times the trilinear grid value at o + t d (no lookup counting).
-__device__ __forceinline__ float density_at(const rtc8x_grid& g, float coeff, V3 o, V3 d, float t)
+__device__ __forceinline__ float density_at(const rtc8x_grid& g, const Medium& m, V3 o, V3 d, float t)
 {
     V3 idx = world_to_index(g, fmaf(t, d.x, o.x), fmaf(t, d.y, o.y), fmaf(t, d.z, o.z));
-    return coeff * trilinear(g, idx);
+    return m.coeff * trilinear(g, m.bricks, idx);
 }
 
 // Density coefficient times the grid value at o + t[s] d for S distances, looked up together.
 template <uint32_t S>
-__device__ __forceinline__ void density_batch(const rtc8x_grid& g, float coeff, V3 o, V3 d, const float (&t)[S],
+__device__ __forceinline__ void density_batch(const rtc8x_grid& g, const Medium& m, V3 o, V3 d, const float (&t)[S],
                                               float (&sig)[S])
 {
     V3 idx[S];
 #pragma unroll
     for (uint32_t s = 0; s < S; ++s) idx[s] = world_to_index(g, fmaf(t[s], d.x, o.x), fmaf(t[s], d.y, o.y), fmaf(t[s], d.z, o.z));
-    trilinear_batch<S>(g, idx, sig);
+    trilinear_batch<S>(g, m.bricks, idx, sig);
 #pragma unroll
-    for (uint32_t s = 0; s < S; ++s) sig[s] = coeff * sig[s];
+    for (uint32_t s = 0; s < S; ++s) sig[s] = m.coeff * sig[s];
 }
 
 __device__ __forceinline__ float sample_density(const rtc8x_grid& g, Medium& m, V3 o, V3 d, float t)
 {
     V3 idx = world_to_index(g, fmaf(t, d.x, o.x), fmaf(t, d.y, o.y), fmaf(t, d.z, o.z));
     m.lookups++;
-    return m.coeff * trilinear(g, idx);
+    return m.coeff * trilinear(g, m.bricks, idx);
 }
 
 // nanovdb::Ray::clip against the float world bbox (util/Ray.h:63-73, 427-455, 512-520)

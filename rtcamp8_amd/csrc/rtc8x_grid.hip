@@ -243,7 +243,7 @@ __global__ void probe_kernel(const rtc8x_grid g, uint32_t n, const float* __rest
     uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= n) return;
     V3 idx = world_to_index(g, xyz[3 * q], xyz[3 * q + 1], xyz[3 * q + 2]);
-    float v = trilinear(g, idx);
+    float v = trilinear(g, has_bricks(g), idx);
     int32_t i = (int32_t)floorf(idx.x), j = (int32_t)floorf(idx.y), k = (int32_t)floorf(idx.z);
     out_ijk[3 * q] = i;
     out_ijk[3 * q + 1] = j;
@@ -421,7 +421,9 @@ struct DeviceArray {
 // would take 2^31 quads (32 GiB) or more, or do not fit the device, go without: lookups then walk the tree.
 rtc8x_status build_bricks(rtc8x_grid& g, uint32_t num_tiles, hipStream_t s)
 {
-    g.leaf_masks = g.lower_masks = g.upper_masks = nullptr;
+    g.bricks = nullptr;
+    g.brick_map = nullptr;
+    g.brick_key = 0;
     const uint64_t d0 = (uint64_t)g.leaf_map_dims[0], d1 = (uint64_t)g.leaf_map_dims[1], d2 = (uint64_t)g.leaf_map_dims[2];
     if (!g.leaf_map || d0 * d1 >= (1u << 24) || d2 >= (1u << 24)) return RTC8X_OK;  // the lookup's 24-bit products
     const size_t n = (size_t)(d0 * d1 * d2);
@@ -451,9 +453,9 @@ rtc8x_status build_bricks(rtc8x_grid& g, uint32_t num_tiles, hipStream_t s)
                        (uint32_t)own, num_tiles, (const uint32_t*)block_of.p, bricks.p);
     RTC8X_HIP(hipGetLastError());
     RTC8X_HIP(hipStreamSynchronize(s));
-    g.lower_masks = reinterpret_cast<const uint64_t*>(bricks.release());
-    g.leaf_masks = reinterpret_cast<const uint64_t*>(map.release());
-    g.upper_masks = reinterpret_cast<const uint64_t*>((uintptr_t)dev::brick_tag(g.lower_masks, g.leaf_masks));
+    g.bricks = reinterpret_cast<const float*>(bricks.release());
+    g.brick_map = map.release();
+    g.brick_key = dev::brick_key(g);
     return RTC8X_OK;
 }
 
@@ -544,11 +546,8 @@ extern "C" rtc8x_status rtc8x_grid_destroy(rtc8x_grid* g)
 try {
     RTC8X_REQUIRE(g != nullptr, "rtc8x_grid_destroy: grid is NULL");
     const void* ptrs[] = {g->root_tiles, g->upper_tables, g->lower_tables, g->leaf_values,     g->tile_values,
-                          g->leaf_origins, g->cell_majorants, g->leaf_map,    g->region_majorants};
-    if (dev::brick_tagged(*g)) {
-        RTC8X_HIP(hipFree(const_cast<uint64_t*>(g->lower_masks)));
-        RTC8X_HIP(hipFree(const_cast<uint64_t*>(g->leaf_masks)));
-    }
+                          g->leaf_origins, g->cell_majorants, g->leaf_map,    g->region_majorants,
+                          g->bricks,     g->brick_map};
     for (const void* p : ptrs)
         if (p) RTC8X_HIP(hipFree(const_cast<void*>(p)));
     std::memset(g, 0, sizeof(*g));
@@ -791,6 +790,9 @@ rtc8x_status upload_host_grid(const rtc8x_grid* h, rtc8x_grid* out, bool keep_ma
     g.region_majorants = nullptr;
     g.leaf_map = nullptr;
     g.leaf_masks = g.lower_masks = g.upper_masks = nullptr;  // host-side activity is not uploaded
+    g.bricks = nullptr;
+    g.brick_map = nullptr;
+    g.brick_key = 0;
     if (h->num_root_tiles > 0 && h->num_leaves > 0) {
         RTC8X_TRY(build_leaf_map(g, nullptr));
         RTC8X_TRY(build_bricks(g, num_tiles_values, nullptr));
@@ -851,6 +853,9 @@ try {
         RTC8X_HIP(hipMemcpy(t.regions.data(), d->region_majorants, nregions, hipMemcpyDeviceToHost));
     }
     rtc8x_grid g = *d;
+    g.bricks = nullptr;
+    g.brick_map = nullptr;
+    g.brick_key = 0;
     g.leaf_map = nullptr;
     for (int a = 0; a < 3; ++a) {
         g.leaf_map_origin[a] = 0;

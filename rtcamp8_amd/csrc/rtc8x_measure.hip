@@ -38,6 +38,7 @@ __global__ void gather_probe_kernel(const rtc8x_grid g, uint32_t steps, uint32_t
     const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t h = mix32(tid * 0x9e3779b9u ^ seed);
     float acc = 0.0f;
+    const bool bricks = dev::has_bricks(g);
     for (uint32_t s = 0; s < steps; ++s) {
         dev::V3 idx[W];
 #pragma unroll
@@ -51,7 +52,7 @@ __global__ void gather_probe_kernel(const rtc8x_grid g, uint32_t steps, uint32_t
                         (float)o[2] + (float)((r >> 16) & 0xffu) * (8.0f / 256.0f)};
         }
         float v[W];
-        dev::trilinear_batch<W>(g, idx, v);
+        dev::trilinear_batch<W>(g, bricks, idx, v);
         float sum = 0.0f;
 #pragma unroll
         for (uint32_t k = 0; k < W; ++k) sum += v[k];
@@ -103,7 +104,7 @@ void march_probe_kernel(const rtc8x_frame_params p, dev::V3 light, uint32_t spp,
     const float coeff = p.density_coeff;
     const float trace_len = 2.0f * p.world_radius;
     dev::Medium med;
-    med.init(p.grid, coeff);
+    med.init(p.grid, coeff, dev::has_bricks(p.grid));
     dev::Seg<RTC8X_TRACKING_LOCAL_MAJORANT> sg;
     dev::Pcg rng;
     rng.state = 0;
@@ -192,7 +193,7 @@ void march_probe_kernel(const rtc8x_frame_params p, dev::V3 light, uint32_t spp,
             tl[0] = tk[0] > t1 ? t : tk[0];
             tl[1] = tk[1] > t1 ? t : tk[1];
             float sig[2];
-            dev::density_batch<2>(p.grid, coeff, o, d, tl, sig);
+            dev::density_batch<2>(p.grid, med, o, d, tl, sig);
             for (int k = 0; k < 2 && event == 0; ++k) {
                 if (tk[k] > t1) {
                     event = 2;

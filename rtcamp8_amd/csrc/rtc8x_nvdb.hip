@@ -38,7 +38,6 @@
 #include <vector>
 
 #include "rtc8x_common.hpp"
-#include "rtc8x_device.hpp"
 
 namespace rtc8x {
 namespace {
@@ -1035,11 +1034,8 @@ try {
     uint32_t num_tiles = 0;
     rtc8x_status st = validate_tables(h, &num_tiles);
     if (st != RTC8X_OK) return st;
-    // tables copied from a device grid by hand keep its lookup bricks in the mask fields: no activity there
-    rtc8x_grid host = *h;
-    if (rtc8x::dev::brick_tagged(host)) host.leaf_masks = host.lower_masks = host.upper_masks = nullptr;
     Encoder e;
-    e.h = &host;
+    e.h = h;
     st = e.plan();
     if (st != RTC8X_OK) return st;
     *size = e.total;

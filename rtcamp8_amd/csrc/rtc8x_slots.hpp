@@ -255,6 +255,7 @@ __device__ __forceinline__ void slots_body(ParamsPtr params, uint32_t W, uint32_
         inv1 = 1.0f / (float)p.grid.region_dims[1];
         inv2 = 1.0f / (float)p.grid.region_dims[2];
     }
+    const bool bricks = has_bricks(p.grid);
     uint32_t paths = 0, vertices = 0, lookups = 0, scatters = 0;
 
     for (;;) {
@@ -318,7 +319,7 @@ __device__ __forceinline__ void slots_body(ParamsPtr params, uint32_t W, uint32_
         const rtc8x_frame_params& p = *(const rtc8x_frame_params*)(ParamsPtr)fresh_params;
         const rtc8x_nrc_buffers& nb = p.nrc;
         Medium med;
-        med.init(p.grid, p.density_coeff);
+        med.init(p.grid, p.density_coeff, bricks);
 
         auto U = [&](uint32_t f) -> uint32_t { return mem.f[f][slot]; };
         auto F = [&](uint32_t f) -> float { return __uint_as_float(mem.f[f][slot]); };
@@ -410,7 +411,7 @@ __device__ __forceinline__ void slots_body(ParamsPtr params, uint32_t W, uint32_
                 }
                 for (;;) {
                     if (st == kPending) {
-                        const float sig = density_at(p.grid, med.coeff, sg.o, sg.d, sg.t);
+                        const float sig = density_at(p.grid, med, sg.o, sg.d, sg.t);
                         looked++;
                         st = kWalking;
                         if (shadow) {

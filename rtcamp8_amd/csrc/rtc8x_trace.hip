@@ -144,7 +144,7 @@ __device__ __forceinline__ void speculate_global(const rtc8x_grid& g, Medium& me
         }
     }
     float sig[S];
-    density_batch<S>(g, med.coeff, sg.o, sg.d, tk, sig);
+    density_batch<S>(g, med, sg.o, sg.d, tk, sig);
     bool accepted = false;
     float t_acc = 0.0f;
     uint64_t st_acc = 0;
@@ -276,7 +276,7 @@ __device__ __forceinline__ void coop_segments(const rtc8x_grid& g, Medium& med, 
             }
             const bool valid = lane < e;
             float sig = 0.0f;
-            if (valid) sig = density_at(g, med.coeff, o, d, tj);
+            if (valid) sig = density_at(g, med, o, d, tj);
             if (track) {
                 const uint64_t acc = __ballot(valid && ua < med.over(sig, maj));
                 if (acc) {
@@ -384,7 +384,7 @@ __device__ __forceinline__ void coop_segments_local(const rtc8x_grid& g, Medium&
                     st_acc = r.state;
                 }
             }
-            const float sig = valid ? density_at(g, med.coeff, c.o, c.d, c.t) : 0.0f;
+            const float sig = valid ? density_at(g, med, c.o, c.d, c.t) : 0.0f;
             const uint32_t e = (uint32_t)__popcll(__ballot(valid));  // the valid lanes are 0 .. e-1
             if (track) {
                 const uint64_t acc = __ballot(valid && ua < med.over(sig, mu));
@@ -492,7 +492,7 @@ __device__ __forceinline__ void trace_body(const rtc8x_frame_params& p, uint32_t
     const float prob_env = (p.sun.enabled && p.env.kind != RTC8X_ENV_NONE) ? 1.0f - p.sun.select_prob : 1.0f;
 
     Medium med;
-    med.init(p.grid, p.density_coeff);
+    med.init(p.grid, p.density_coeff, has_bricks(p.grid));
     uint32_t paths = 0, vertices = 0, scatters = 0;
 
     Lane L;
@@ -941,7 +941,7 @@ __device__ __forceinline__ void trace_body(const rtc8x_frame_params& p, uint32_t
                 const int r2 = sg.advance(p.grid, med, L.rng, mu_second, region_table);
                 const float tk[2] = {t_first, r2 == kAdvanceCollision ? sg.t : t_first};
                 float sig[2];
-                density_batch<2>(p.grid, med.coeff, sg.o, sg.d, tk, sig);
+                density_batch<2>(p.grid, med, sg.o, sg.d, tk, sig);
                 med.lookups++;
                 if (track && u_first < med.over(sig[0], mu_first)) {
                     sg.t = t_first;

@@ -66,3 +66,76 @@ def test_brick_lookups_match_the_tree(kind):
             assert sizes[0] == sizes[1] > 0
     finally:
         call("rtc8x_grid_destroy", C.byref(dg))
+
+
+def _probe(grid, pts):
+    from rtcamp8_amd._lib import call
+    from rtcamp8_amd.device import DeviceBuffer
+
+    n = len(pts)
+    d = [DeviceBuffer.from_array(pts), DeviceBuffer(12 * n), DeviceBuffer(12 * n), DeviceBuffer(4 * n)]
+    call("rtc8x_grid_probe", C.byref(grid), n, *[C.c_void_p(b.ptr) for b in d], None)
+    return d[3].download(np.float32, n)
+
+
+def _oracle_probe(grid, pts):
+    n = len(pts)
+    ijk, off, val = np.empty(3 * n, np.int32), np.empty(3 * n, np.uint32), np.empty(n, np.float32)
+    oracle().oracle_grid_probe(C.byref(grid), n, ptr(pts), ptr(ijk), ptr(off), ptr(val))
+    return val
+
+
+@pytest.mark.parametrize("table", ["leaf_values", "tile_values"])
+def test_lookups_follow_tables_put_into_a_copy(table):
+    """A copy of a device grid with another table of values is looked up in that table, not in bricks that
+    hold the former one's."""
+    from rtcamp8_amd import _abi
+    from rtcamp8_amd._lib import call
+    from rtcamp8_amd.device import DeviceBuffer
+
+    hg, origins = _grid("tiles")
+    rng = np.random.default_rng(14)
+    pts = np.ascontiguousarray(origins[rng.integers(0, len(origins), 4000)] + rng.uniform(-18.0, 26.0, (4000, 3)), np.float32)
+    dg = _abi.Grid()
+    call("rtc8x_grid_upload", C.byref(hg.grid), C.byref(dg))
+    try:
+        key = "values" if table == "leaf_values" else "tiles"
+        other = np.ascontiguousarray(1.0 - hg.arrays[key].reshape(-1), np.float32)
+        if key == "tiles":
+            other[0] = hg.arrays[key][0]  # the background stays tile 0
+        d = DeviceBuffer.from_array(np.append(other, np.float32(0.0)))  # one float of padding
+        copy = _abi.Grid.from_buffer_copy(dg)
+        setattr(copy, table, d.ptr)
+        host = _abi.Grid.from_buffer_copy(hg.grid)
+        setattr(host, table, other.ctypes.data)
+        assert np.array_equal(_probe(copy, pts).view(np.uint32), _oracle_probe(host, pts).view(np.uint32))
+        assert np.array_equal(_probe(dg, pts).view(np.uint32), _oracle_probe(hg.grid, pts).view(np.uint32))
+    finally:
+        call("rtc8x_grid_destroy", C.byref(dg))
+
+
+def test_the_mask_fields_are_the_callers():
+    """The library neither uses nor needs a device grid's host-only mask fields: with them cleared the grid is
+    looked up as before and destroyed whole."""
+    import torch
+
+    from rtcamp8_amd import _abi
+    from rtcamp8_amd._lib import call
+
+    desc = _abi.FbmDesc()
+    desc.resolution, desc.octaves, desc.seed = 128, 4, 5
+    desc.base_frequency, desc.lacunarity, desc.gain, desc.contrast = 4.0, 2.0, 0.5, 1.0
+
+    def cycle():
+        dg = _abi.Grid()
+        call("rtc8x_grid_build_fbm", C.byref(desc), C.byref(dg), None)
+        assert not dg.leaf_masks and not dg.lower_masks and not dg.upper_masks
+        assert dg.bricks and dg.brick_map
+        dg.leaf_masks = dg.lower_masks = dg.upper_masks = None
+        call("rtc8x_grid_destroy", C.byref(dg))
+
+    cycle()
+    free = torch.cuda.mem_get_info()[0]
+    for _ in range(4):  # the bricks take 36 MB
+        cycle()
+    assert torch.cuda.mem_get_info()[0] >= free - (16 << 20)
