@@ -139,3 +139,72 @@ def test_the_mask_fields_are_the_callers():
     for _ in range(4):  # the bricks take 36 MB
         cycle()
     assert torch.cuda.mem_get_info()[0] >= free - (16 << 20)
+
+
+@pytest.mark.parametrize("kind", ["one_leaf", "across_roots", "tiles"])
+@pytest.mark.parametrize("leaf_map", [True, False])
+def test_lookups_without_bricks_match_the_tree(kind, leaf_map):
+    from rtcamp8_amd import _abi
+    from rtcamp8_amd._lib import call
+
+    hg, origins = _grid(kind)
+    rng = np.random.default_rng(13)
+    n = 20000
+    pts = origins[rng.integers(0, len(origins), n)] + rng.uniform(-18.0, 26.0, (n, 3))
+    pts[: n // 2] = np.round(pts[: n // 2] / 8.0) * 8.0 - rng.choice([0.0, 0.25, 0.5, 1.0, 7.5], (n // 2, 3))
+    pts = np.ascontiguousarray(pts, np.float32)
+    dg = _abi.Grid()
+    call("rtc8x_grid_upload", C.byref(hg.grid), C.byref(dg))
+    try:
+        bare = _abi.Grid.from_buffer_copy(dg)
+        bare.bricks = None
+        if not leaf_map:
+            bare.leaf_map = None
+        assert np.array_equal(_probe(bare, pts).view(np.uint32), _oracle_probe(hg.grid, pts).view(np.uint32))
+    finally:
+        call("rtc8x_grid_destroy", C.byref(dg))
+
+
+@pytest.mark.parametrize("tracking", [0, 1])
+def test_frames_without_bricks(tracking):
+    """Frames of the plain and the cache-rendering entry and training records: the same bits with and without."""
+    from rtcamp8_amd import _abi
+    from rtcamp8_amd import scene as sc
+    from rtcamp8_amd._lib import call
+    from rtcamp8_amd.nrc import NrcRenderer
+    from rtcamp8_amd.tracer import PathTracer
+
+    cfg = sc.CONFIGS["sparse512"].with_(width=75, height=41, tracking=tracking, sky_width=64, sky_height=32,
+                                        fbm=sc.FbmConfig(resolution=128, seed=0x5EED0007, sparse=True,
+                                                         active_leaf_fraction=0.25))
+    s = sc.DeviceScene(cfg)
+    npx = cfg.width * cfg.height
+    got = []
+    for bricks in (True, False):
+        t, r = PathTracer(s), NrcRenderer(s, samples_per_launch=2)
+
+        def params(owner):
+            p = owner.params()
+            if not bricks:
+                p.grid.bricks = None
+            return p
+
+        for _ in range(2):
+            t.trace(2, params(t))
+        p = params(r)
+        p.nrc.num_samples = 2
+        call("rtc8x_trace", None, C.byref(p), _abi.ENTRY_PATH_TRACE_WITH_NRC, 2)
+        out = [t.accum.download(np.uint64, 3 * npx), t.rng.download(np.uint64, npx), t.stats.download(np.uint64, 4),
+               r.buffers.inference_terminals.download(np.uint32), r.buffers.per_frame_contribution.download(np.uint32)]
+        p = params(r)
+        call("rtc8x_nrc_prepare", None, C.byref(p), 1)
+        call("rtc8x_trace", None, C.byref(p), _abi.ENTRY_GENERATE_TRAINING_DATA, 1)
+        n = int(r.buffers.num_training_data.download(np.uint32, 2)[p.nrc.nrc_buffer_index])
+        out += [np.array([n]), r.buffers.train_queries[0].download(np.uint32, 14 * min(n, 1000)), r.rng.download(np.uint64, npx)]
+        got.append(out)
+        t.close()
+        r.close()
+    s.close()
+    assert got[0][5][0] > 0  # there were training records
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
