@@ -198,8 +198,9 @@ typedef struct rtc8x_grid {
      * stencil, 9,216 bytes per 8^3 block that is not inside one tile, and one u32 per block of the leaf map;
      * about 4.5 times the bytes of leaf_values.  A cache of the tables: lookups without them give the same
      * values.  The layout is the library's own.  brick_key names the tables they were filled from; a grid
-     * with other leaf_values, tile_values or leaf_map is looked up without them.  Values changed in place need
-     * new bricks. */
+     * with other leaf_values, tile_values or leaf_map is looked up without them.  A new grid gets them where they
+     * take less than 32 GiB and at most an eighth of the device's free memory; rtc8x_grid_build_bricks bounds
+     * them otherwise, frees them, or fills them anew after values changed in place.  NULL: no bricks. */
     const float* bricks;
     const uint32_t* brick_map;
     uint64_t brick_key;
@@ -237,6 +238,11 @@ rtc8x_status rtc8x_grid_destroy(rtc8x_grid* grid);
  * tighter majorants); callers tune it per volume.  No counterpart in the reference, which tracks with
  * the global majorant only (renderer_scene.cpp:499-511). */
 rtc8x_status rtc8x_grid_build_regions(rtc8x_grid* grid, uint32_t region_cells);
+/* Frees a device grid's lookup bricks and builds them anew from its tables where they and their map take at
+ * most max_bytes (0: none), fit the device and take less than 32 GiB; grid->bricks is NULL otherwise.  The
+ * results of lookups are the same either way; the trackers run up to half again as long without.
+ * Synchronises the device. */
+rtc8x_status rtc8x_grid_build_bricks(rtc8x_grid* grid, uint64_t max_bytes);
 /* Parity probe: for n world-space points, the index coordinate, node offsets and trilinear value
  * exactly as the tracer computes them.  out_ijk[3n], out_offsets[3n] = (upper, lower, leaf) offsets,
  * out_value[n]; all device pointers. */

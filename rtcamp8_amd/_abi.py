@@ -381,6 +381,7 @@ PROTOTYPES = {
     "rtc8x_grid_upload": (_S, [C.POINTER(Grid), C.POINTER(Grid)]),
     "rtc8x_grid_destroy": (_S, [C.POINTER(Grid)]),
     "rtc8x_grid_build_regions": (_S, [C.POINTER(Grid), C.c_uint32]),
+    "rtc8x_grid_build_bricks": (_S, [C.POINTER(Grid), C.c_uint64]),
     "rtc8x_grid_probe": (_S, [C.POINTER(Grid), C.c_uint32, _P, _P, _P, _P, _P]),
     "rtc8x_nvdb_list": (_S, [_P, C.c_size_t, C.POINTER(NvdbGridInfo), C.c_uint32, C.POINTER(C.c_uint32)]),
     "rtc8x_nanovdb_decode": (_S, [_P, C.c_size_t, C.POINTER(Grid)]),

@@ -151,17 +151,28 @@ __device__ __forceinline__ bool same_tile_block(const rtc8x_grid& g, size_t q, i
     return same;
 }
 
-// Blocks with a brick of their own per 256-lane workgroup.
-__global__ __launch_bounds__(256) void brick_count_kernel(const rtc8x_grid g, size_t n, uint32_t* __restrict__ sums)
+// Per 256-lane workgroup: blocks with a brick of their own, and one more than the largest tile index that the
+// others name (0: none do).
+__global__ __launch_bounds__(256) void brick_count_kernel(const rtc8x_grid g, size_t n, uint32_t* __restrict__ sums,
+                                                          uint32_t* __restrict__ tiles)
 {
-    __shared__ uint32_t part[4];
+    __shared__ uint32_t part[4], top[4];
     const size_t q = (size_t)blockIdx.x * 256 + threadIdx.x;
     int32_t o[3];
     uint32_t e;
-    const uint64_t own = __ballot(q < n && !same_tile_block(g, q, o, e));
-    if ((threadIdx.x & 63u) == 0) part[threadIdx.x >> 6] = (uint32_t)__popcll(own);
+    const bool shared = q < n && same_tile_block(g, q, o, e);
+    const uint64_t own = __ballot(q < n && !shared);
+    uint32_t t = shared ? (e & ~RTC8X_TILE_BIT) + 1u : 0u;
+    for (int k = 32; k > 0; k >>= 1) t = max(t, (uint32_t)__shfl_xor((int)t, k, 64));
+    if ((threadIdx.x & 63u) == 0) {
+        part[threadIdx.x >> 6] = (uint32_t)__popcll(own);
+        top[threadIdx.x >> 6] = t;
+    }
     __syncthreads();
-    if (threadIdx.x == 0) sums[blockIdx.x] = part[0] + part[1] + part[2] + part[3];
+    if (threadIdx.x == 0) {
+        sums[blockIdx.x] = part[0] + part[1] + part[2] + part[3];
+        tiles[blockIdx.x] = max(max(top[0], top[1]), max(top[2], top[3]));
+    }
 }
 
 // The map's entries: the first quad of each block's brick.  Two quads per tile value come first, then the
@@ -417,9 +428,10 @@ struct DeviceArray {
     }
 };
 
-// The lookup bricks of a grid with a leaf map (rtc8x_device.hpp); num_tiles tile values.  Grids whose bricks
-// would take 2^31 quads (32 GiB) or more, or do not fit the device, go without: lookups then walk the tree.
-rtc8x_status build_bricks(rtc8x_grid& g, uint32_t num_tiles, hipStream_t s)
+// The lookup bricks of a grid with a leaf map (rtc8x_device.hpp).  Grids whose bricks would take 2^31 quads
+// (32 GiB) or more, or more than max_bytes with their map, or do not fit the device, go without: lookups then
+// read the leaves.
+rtc8x_status build_bricks(rtc8x_grid& g, uint64_t max_bytes, hipStream_t s)
 {
     g.bricks = nullptr;
     g.brick_map = nullptr;
@@ -428,23 +440,26 @@ rtc8x_status build_bricks(rtc8x_grid& g, uint32_t num_tiles, hipStream_t s)
     if (!g.leaf_map || d0 * d1 >= (1u << 24) || d2 >= (1u << 24)) return RTC8X_OK;  // the lookup's 24-bit products
     const size_t n = (size_t)(d0 * d1 * d2);
     const uint32_t groups = (uint32_t)((n + 255) / 256);
+    if (n * sizeof(uint32_t) > max_bytes) return RTC8X_OK;
     DeviceArray<uint32_t> sums, map, block_of;
     DeviceArray<float4> bricks;
-    if (!sums.alloc(groups) || !map.alloc(n)) return RTC8X_OK;
-    hipLaunchKernelGGL(dev::brick_count_kernel, dim3(groups), dim3(256), 0, s, g, n, sums.p);
+    if (!sums.alloc(2 * (size_t)groups)) return RTC8X_OK;
+    hipLaunchKernelGGL(dev::brick_count_kernel, dim3(groups), dim3(256), 0, s, g, n, sums.p, sums.p + groups);
     RTC8X_HIP(hipGetLastError());
-    std::vector<uint32_t> base(groups);
-    RTC8X_HIP(hipMemcpyAsync(base.data(), sums.p, groups * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    std::vector<uint32_t> base(2 * (size_t)groups);
+    RTC8X_HIP(hipMemcpyAsync(base.data(), sums.p, base.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     RTC8X_HIP(hipStreamSynchronize(s));
     uint64_t own = 0;
-    for (uint32_t& b : base) {
-        const uint32_t c = b;
-        b = (uint32_t)own;
+    uint32_t num_tiles = 0;
+    for (uint32_t i = 0; i < groups; ++i) {
+        const uint32_t c = base[i];
+        base[i] = (uint32_t)own;
         own += c;
+        num_tiles = std::max(num_tiles, base[groups + i]);
     }
     const uint64_t quads = 2 * (uint64_t)num_tiles + own * dev::kBrickQuads;
-    if (quads >= dev::kSharedBrick) return RTC8X_OK;
-    if (!block_of.alloc(own) || !bricks.alloc(quads)) return RTC8X_OK;
+    if (quads >= dev::kSharedBrick || quads * sizeof(float4) + n * sizeof(uint32_t) > max_bytes) return RTC8X_OK;
+    if (!map.alloc(n) || !block_of.alloc(own) || !bricks.alloc(quads)) return RTC8X_OK;
     RTC8X_HIP(hipMemcpyAsync(sums.p, base.data(), groups * sizeof(uint32_t), hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL(dev::brick_map_kernel, dim3(groups), dim3(256), 0, s, g, n, num_tiles, (const uint32_t*)sums.p, map.p,
                        block_of.p);
@@ -456,6 +471,16 @@ rtc8x_status build_bricks(rtc8x_grid& g, uint32_t num_tiles, hipStream_t s)
     g.bricks = reinterpret_cast<const float*>(bricks.release());
     g.brick_map = map.release();
     g.brick_key = dev::brick_key(g);
+    return RTC8X_OK;
+}
+
+// What a new grid's bricks may take unasked: an eighth of the device's free memory (36 GB of an idle card's), so
+// that a volume leaves a card that it shares to the others.
+rtc8x_status default_brick_bytes(uint64_t* bytes)
+{
+    size_t free_bytes = 0, total = 0;
+    RTC8X_HIP(hipMemGetInfo(&free_bytes, &total));
+    *bytes = free_bytes / 8;
     return RTC8X_OK;
 }
 
@@ -541,6 +566,20 @@ try {
     return RTC8X_OK;
 }
 RTC8X_CATCH_ALL("rtc8x_grid_build_regions")
+
+extern "C" rtc8x_status rtc8x_grid_build_bricks(rtc8x_grid* g, uint64_t max_bytes)
+try {
+    RTC8X_REQUIRE(g != nullptr, "rtc8x_grid_build_bricks: grid is NULL");
+    RTC8X_HIP(hipDeviceSynchronize());
+    const void* ptrs[] = {g->bricks, g->brick_map};
+    g->bricks = nullptr;
+    g->brick_map = nullptr;
+    g->brick_key = 0;
+    for (const void* p : ptrs)
+        if (p) RTC8X_HIP(hipFree(const_cast<void*>(p)));
+    return build_bricks(*g, max_bytes, nullptr);
+}
+RTC8X_CATCH_ALL("rtc8x_grid_build_bricks")
 
 extern "C" rtc8x_status rtc8x_grid_destroy(rtc8x_grid* g)
 try {
@@ -697,7 +736,9 @@ try {
     RTC8X_HIP(hipGetLastError());
     RTC8X_HIP(hipStreamSynchronize(s));
     RTC8X_TRY(build_leaf_map(g, s));
-    RTC8X_TRY(build_bricks(g, 1, s));
+    uint64_t brick_bytes = 0;
+    RTC8X_TRY(default_brick_bytes(&brick_bytes));
+    RTC8X_TRY(build_bricks(g, brick_bytes, s));
     RTC8X_TRY(build_majorant_tables(g, 0, s));
     *out = g;
     return RTC8X_OK;
@@ -795,7 +836,9 @@ rtc8x_status upload_host_grid(const rtc8x_grid* h, rtc8x_grid* out, bool keep_ma
     g.brick_key = 0;
     if (h->num_root_tiles > 0 && h->num_leaves > 0) {
         RTC8X_TRY(build_leaf_map(g, nullptr));
-        RTC8X_TRY(build_bricks(g, num_tiles_values, nullptr));
+        uint64_t brick_bytes = 0;
+        RTC8X_TRY(default_brick_bytes(&brick_bytes));
+        RTC8X_TRY(build_bricks(g, brick_bytes, nullptr));
     }
     RTC8X_TRY(build_majorant_tables(g, 0, nullptr));
     *out = g;

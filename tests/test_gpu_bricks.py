@@ -208,3 +208,42 @@ def test_frames_without_bricks(tracking):
     assert got[0][5][0] > 0  # there were training records
     for a, b in zip(*got):
         assert np.array_equal(a, b)
+
+
+def test_bricks_within_a_bound():
+    """rtc8x_grid_build_bricks: none, none within too few bytes, all within enough, filled from the values that
+    the tables hold by then; the same lookups throughout."""
+    import torch
+
+    from rtcamp8_amd import _abi
+    from rtcamp8_amd._lib import call
+
+    hg, origins = _grid("tiles")
+    rng = np.random.default_rng(15)
+    pts = np.ascontiguousarray(origins[rng.integers(0, len(origins), 5000)] + rng.uniform(-18.0, 26.0, (5000, 3)), np.float32)
+    dg = _abi.Grid()
+    call("rtc8x_grid_upload", C.byref(hg.grid), C.byref(dg))
+    try:
+        assert dg.bricks
+        ref = _oracle_probe(hg.grid, pts).view(np.uint32)
+        own = 9216 * len(origins)  # the leaves' own bricks, without those of the blocks beside them
+        for most, have in ((0, False), (own, False), (16 * own, True), (0, False), (1 << 40, True)):
+            call("rtc8x_grid_build_bricks", C.byref(dg), most)
+            assert bool(dg.bricks) == have and bool(dg.brick_map) == have, most
+            assert np.array_equal(_probe(dg, pts).view(np.uint32), ref), most
+        values = np.ascontiguousarray(2.0 * hg.arrays["values"].reshape(-1), np.float32)
+        call("rtc8x_memcpy_htod", C.c_void_p(dg.leaf_values), values.ctypes.data_as(C.c_void_p), values.nbytes)
+        call("rtc8x_grid_build_bricks", C.byref(dg), 1 << 40)
+        host = _abi.Grid.from_buffer_copy(hg.grid)
+        host.leaf_values = values.ctypes.data
+        assert np.array_equal(_probe(dg, pts).view(np.uint32), _oracle_probe(host, pts).view(np.uint32))
+    finally:
+        call("rtc8x_grid_destroy", C.byref(dg))
+    desc = _abi.FbmDesc()
+    desc.resolution, desc.octaves, desc.seed = 128, 4, 5
+    desc.base_frequency, desc.lacunarity, desc.gain, desc.contrast = 4.0, 2.0, 0.5, 1.0
+    call("rtc8x_grid_build_fbm", C.byref(desc), C.byref(dg), None)
+    free = torch.cuda.mem_get_info()[0]
+    call("rtc8x_grid_build_bricks", C.byref(dg), 0)
+    assert torch.cuda.mem_get_info()[0] >= free + (30 << 20)  # 36 MB of bricks
+    call("rtc8x_grid_destroy", C.byref(dg))
