@@ -411,8 +411,12 @@ struct Medium {
         normal = majorant >= 0x1p-40f && majorant <= 0x1p40f &&
                  (!g.region_majorants || (unit >= 0x1p-40f && unit <= 0x1p33f));
     }
-    // a over a majorant
-    __device__ __forceinline__ float over(float a, float mu) const { return normal ? div_normal(a, mu) : a / mu; }
+    // a over a majorant.  Voxels may be infinite or as large as floats are, whatever the majorants: those are
+    // divided in full, and no others (the fast division makes a NaN of infinity).
+    __device__ __forceinline__ float over(float a, float mu) const
+    {
+        return normal && fabsf(a) <= 0x1p40f ? div_normal(a, mu) : a / mu;
+    }
 };
 
 // Density coefficient times the trilinear grid value at o + t d (no lookup counting).
