@@ -342,7 +342,7 @@ def multi_instance_leg(steps: int, stream):
             "entry": "PATH_TRACE_WITH_NRC, 1 spp per instance",
             "one_launch_per_instance_ms": seq_ms, "one_launch_per_instance_tuned_ms": seq_tuned_ms,
             "batched_autotuned_ms": tuned_ms, "batched_by_pixels_ms": pixel_ms,
-            "autotuned": [{"event_eighths": k[0], "tile": batch.TILE_SHAPES[k[1]], "share_ms": sh}
+            "autotuned": [{"tile": batch.TILE_SHAPES[k[1]], "share_ms": sh}
                           for k, sh in zip(solo_knobs, solo_shares)],
             "batch_choice": choice,
             "autotune_seconds": tune_s,

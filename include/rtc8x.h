@@ -581,11 +581,9 @@ typedef struct rtc8x_frame_params {
     const uint32_t* work_order;
     rtc8x_nrc_buffers nrc;
     /* Scheduling knobs (no counterpart in the reference; results do not depend on them), 0 = default:
-     * event_eighths, 1..8, in batched launches and GENERATE_TRAINING_DATA: a wavefront runs its parked lanes'
-     * vertex events once that many eighths of its active lanes are parked (default 5 for PATH_TRACE and
-     * PATH_TRACE_WITH_NRC with local-majorant tracking, 4 with the global majorant, 3 for
-     * GENERATE_TRAINING_DATA); tile_shape: the pixel tiles lanes take without a work order, 0 = 8x8 (default),
-     * 1 = 16x4, 2 = 32x2, 3 = 4x16. */
+     * event_eighths, 1..8, in GENERATE_TRAINING_DATA: a wavefront runs its parked lanes' vertex events once that
+     * many eighths of its active lanes are parked (default 3); tile_shape: the pixel tiles that paths start from
+     * without a work order, 0 = 8x8 (default), 1 = 16x4, 2 = 32x2, 3 = 4x16. */
     uint32_t event_eighths;
     uint32_t tile_shape;
 } rtc8x_frame_params;

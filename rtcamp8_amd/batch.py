@@ -2,8 +2,7 @@
 
 An instance is a PathTracer (plain entry) or an NrcRenderer (the NRC render entry), each with its own
 scene, image and buffers.  `autotune` times every instance's own launch under each candidate setting of
-the tracer's scheduling knobs (the event threshold: how many eighths of a wavefront's active lanes park
-before their vertex events run; and the shape of the 64-pixel tiles lanes take), keeps each instance's
+the tracer's scheduling knobs (the shape of the 64-pixel tiles that paths start from), keeps each instance's
 fastest setting, and returns the fastest times as the workgroup shares of the batched launch, so that
 the instances finish together; `pick_batch_setting` then checks those choices against the plain ones on
 the batched launch.  The knobs change the schedule, never the results."""
@@ -63,8 +62,9 @@ def render_nrc(renderers: Sequence[NrcRenderer], samples: Sequence[int], shares=
         r.stats.inference_queries += nq
 
 
-# (event_eighths, tile_shape) candidates: events from 2/8 to 5/8 of the active lanes; 8x8, 16x4, 4x16 tiles
-KNOB_CANDIDATES = [(ev, shape) for ev in (2, 3, 4, 5) for shape in (0, 1, 3)]
+# (event_eighths, tile_shape) candidates: 8x8, 16x4, 4x16 tiles.  The full-image entries have no event threshold;
+# four candidates of it would be one launch timed four times.
+KNOB_CANDIDATES = [(0, shape) for shape in (0, 1, 3)]
 TILE_SHAPES = {0: "8x8", 1: "16x4", 2: "32x2", 3: "4x16"}
 
 
@@ -103,7 +103,7 @@ def pick_batch_setting(launch_batch, settings, repeats: int = 3, stream=None):
     """The autotuner's last step, on the batched launch itself: times launch_batch(shares, knobs) for
     every candidate (shares, knobs) in `settings` (the best of `repeats`, after one untimed launch) and
     returns (shares, knobs, ms) of the fastest.  Solo launch times make shares only approximately: in the
-    batch the instances share the device and wavefronts move on to unfinished instances, so the solo
+    batch the instances share the device and workgroups move on to unfinished instances, so the solo
     choices are checked against the plain ones (shares by pixels, default knobs) there."""
     best = None
     for shares, knobs in settings:

@@ -204,8 +204,11 @@ struct RegionWalk {
 // parameters of every kind together spill (130 SGPRs, a quarter of the VALU instructions to move them).
 typedef const __attribute__((address_space(4))) rtc8x_frame_params* ParamsPtr;
 
+// One image by workgroup wg of its wgs; helper: a workgroup of another image of the batch, which takes pixels
+// from this one's work counter only.
 template <int ENTRY, int TRACKING, uint32_t REGION_BYTES, uint32_t WAVES>
 __device__ __forceinline__ void slots_body(ParamsPtr params, uint32_t W, uint32_t H, uint32_t num_samples, uint32_t ctr,
+                                           uint32_t wg, uint32_t wgs, bool helper,
                                            SlotMem<ENTRY, TRACKING, REGION_BYTES, WAVES>& mem)
 {
     using Lay = SlotLayout<ENTRY, TRACKING, REGION_BYTES>;
@@ -226,8 +229,17 @@ __device__ __forceinline__ void slots_body(ParamsPtr params, uint32_t W, uint32_
     // each workgroup in turn: the counter's atomics go through one address, and three thousand wavefronts
     // asking at once waited 30 us for their first pixel.  (With more pixels than slots, dealing out the first
     // ones costs more than the wait: 30.2 against 29.2 ms per global-majorant frame of the 512^3 cloud.)
-    const uint32_t share = (total + gridDim.x - 1) / gridDim.x;
+    const uint32_t share = (total + wgs - 1) / wgs;
     const bool few = share < Lay::kSlots;
+    if (helper) {
+        // nothing to do here unless pixels are counted out and some are left
+        if (few) return;
+        if (threadIdx.x == 0) mem.active = __hip_atomic_load(&g_work_counter[ctr], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        const bool left = mem.active < total;
+        __syncthreads();
+        if (!left) return;
+    }
     const uint32_t n0 = few ? (share + kDealt - 1) / kDealt * kDealt : Lay::kSlots;
     const uint32_t waves = blockDim.x >> 6;
     for (uint32_t i = threadIdx.x; i < kWorkKinds * 64u; i += blockDim.x) {
@@ -551,7 +563,7 @@ __device__ __forceinline__ void slots_body(ParamsPtr params, uint32_t W, uint32_
                 }
             };
             if (need && few && pix == kPixNone) {
-                const uint32_t w = (slot / kDealt * gridDim.x + blockIdx.x) * kDealt + slot % kDealt;
+                const uint32_t w = (slot / kDealt * wgs + wg) * kDealt + slot % kDealt;
                 if (w < total) take(w);
             }
             if (need && few) {
@@ -827,7 +839,35 @@ __global__ __launch_bounds__(64 * WAVES) void slots_kernel(const rtc8x_frame_par
     (void)p;  // the first kernel argument, read through the argument segment
     __shared__ SlotMem<ENTRY, TRACKING, REGION_BYTES, WAVES> mem;
     slots_body<ENTRY, TRACKING, REGION_BYTES, WAVES>((ParamsPtr)__builtin_amdgcn_kernarg_segment_ptr(), W, H, num_samples, ctr,
-                                                     mem);
+                                                     blockIdx.x, gridDim.x, false, mem);
+}
+
+// Several images (instances: their own volume, camera, sky, buffers and, with the NRC entry, cache buffers) in one
+// persistent launch.  Workgroup b starts on the instance whose workgroup range [wg_end[i-1], wg_end[i]) holds b
+// (the ranges are the caller's shares of the device, rtc8x_trace_batch); once its instance's last paths are
+// done it moves on to the following instances and helps with what is left of them.
+struct BatchArgs {
+    const rtc8x_frame_params* params;  // device copy, count entries
+    uint32_t count, ctr;               // instance i counts its work at g_work_counter[ctr + i]
+    uint32_t wg_end[kMaxBatch];
+    uint32_t num_samples[kMaxBatch];
+};
+
+template <int ENTRY, int TRACKING, uint32_t REGION_BYTES, uint32_t WAVES>
+__global__ __launch_bounds__(64 * WAVES) void slots_batch_kernel(const BatchArgs b)
+{
+    __shared__ SlotMem<ENTRY, TRACKING, REGION_BYTES, WAVES> mem;
+    uint32_t first = 0;
+    while (first + 1 < b.count && blockIdx.x >= b.wg_end[first]) ++first;
+    for (uint32_t k = 0; k < b.count; ++k) {
+        const uint32_t inst = first + k < b.count ? first + k : first + k - b.count;
+        const uint32_t wg0 = inst ? b.wg_end[inst - 1] : 0u;
+        const rtc8x_frame_params* pp = b.params + inst;
+        slots_body<ENTRY, TRACKING, REGION_BYTES, WAVES>((ParamsPtr)(uint64_t)pp, pp->image_width, pp->image_height,
+                                                         b.num_samples[inst], b.ctr + inst, blockIdx.x - wg0,
+                                                         b.wg_end[inst] - wg0, k != 0, mem);
+        __syncthreads();  // the LDS is free for the next instance
+    }
 }
 
 }  // namespace dev

@@ -1034,33 +1034,6 @@ void wavefront_kernel(const rtc8x_frame_params p, uint32_t launch_w,
     }
 }
 
-// Several images (instances: their own volume, camera, sky, buffers and, with the NRC entry, cache
-// buffers) in one persistent launch.  Workgroup b starts on the instance whose workgroup range
-// [wg_end[i-1], wg_end[i]) holds b (the ranges are the caller's shares of the device,
-// rtc8x_trace_batch) and takes pixels from that instance's work counter; a wavefront that has
-// finished its instance's last pixels moves on to the following instances and helps with what is left
-// of them.  The instance is uniform over a wavefront, so its frame parameters are read with scalar
-// loads, as a single launch reads its kernel arguments.
-struct BatchArgs {
-    const rtc8x_frame_params* params;  // device copy, count entries
-    uint32_t count, slot;              // instance i counts its work at g_work_counter[slot + i]
-    uint32_t wg_end[kMaxBatch];
-    uint32_t num_samples[kMaxBatch];
-};
-
-template <int ENTRY, int TRACKING>
-__global__ __launch_bounds__(256) void batch_kernel(const BatchArgs b)
-{
-    uint32_t first = 0;
-    while (first + 1 < b.count && blockIdx.x >= b.wg_end[first]) ++first;
-    for (uint32_t k = 0; k < b.count; ++k) {
-        const uint32_t inst = first + k < b.count ? first + k : first + k - b.count;
-        const rtc8x_frame_params* __restrict__ pp = b.params + inst;
-        trace_body<ENTRY, TRACKING>(*pp, pp->image_width, pp->image_height, b.num_samples[inst], b.slot + inst,
-                                    nullptr, nullptr, TrainStage{}, pp->grid.region_majorants);
-    }
-}
-
 __global__ void reset_counters_kernel(uint32_t slot, uint32_t count)
 {
     if (threadIdx.x < count) g_work_counter[slot + threadIdx.x] = 0u;
@@ -1430,6 +1403,11 @@ hipError_t launch(const rtc8x_frame_params& p, uint32_t w, uint32_t h, uint32_t 
 // the others would only look for work (256 x 256, 4 samples: 0.71 ms with 8, 0.74 with 6, 0.75 with 12, 0.85
 // with 16 wavefronts).
 constexpr uint32_t kSlotWaves = 16, kSlotWavesFew = 8;
+inline bool few_paths(uint64_t pixels, uint32_t workgroups) { return pixels <= 64ull * kSlotWavesFew * workgroups; }
+inline uint32_t region_bytes(const rtc8x_grid& g)
+{
+    return ((uint32_t)g.region_dims[0] * (uint32_t)g.region_dims[1] * (uint32_t)g.region_dims[2] + 15u) & ~15u;
+}
 template <int ENTRY, int TRACKING, uint32_t REGION_BYTES>
 hipError_t launch_slots(const rtc8x_frame_params& p, uint32_t num_samples, hipStream_t stream)
 {
@@ -1440,8 +1418,7 @@ hipError_t launch_slots(const rtc8x_frame_params& p, uint32_t num_samples, hipSt
     e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(reset_counter_kernel, dim3(1), dim3(1), 0, stream, ctr);
-    const uint64_t share = ((uint64_t)p.image_width * p.image_height + cus - 1) / cus;
-    const uint32_t waves = share <= 64 * kSlotWavesFew ? kSlotWavesFew : kSlotWaves;
+    const uint32_t waves = few_paths((uint64_t)p.image_width * p.image_height, (uint32_t)cus) ? kSlotWavesFew : kSlotWaves;
     hipLaunchKernelGGL((slots_kernel<ENTRY, TRACKING, REGION_BYTES, kSlotWaves>), dim3((uint32_t)cus), dim3(64 * waves), 0,
                        stream, p, p.image_width, p.image_height, num_samples, ctr);
     return hipGetLastError();
@@ -1454,47 +1431,62 @@ hipError_t launch_slots_tracking(const rtc8x_frame_params& p, uint32_t num_sampl
 {
     if (p.tracking != RTC8X_TRACKING_LOCAL_MAJORANT)
         return launch_slots<ENTRY, RTC8X_TRACKING_GLOBAL_MAJORANT, 0>(p, num_samples, stream);
-    const uint32_t regions = ((uint32_t)p.grid.region_dims[0] * (uint32_t)p.grid.region_dims[1] * (uint32_t)p.grid.region_dims[2] + 15u) & ~15u;
-    if (regions <= kSmallRegions)
+    if (region_bytes(p.grid) <= kSmallRegions)
         return launch_slots<ENTRY, RTC8X_TRACKING_LOCAL_MAJORANT, kSmallRegions>(p, num_samples, stream);
     return launch_slots<ENTRY, RTC8X_TRACKING_LOCAL_MAJORANT, RTC8X_MAX_REGIONS>(p, num_samples, stream);
 }
 
-// One persistent launch over several instances; shares[i] is instance i's part of the device's
-// workgroups (each gets at least one).
-template <int ENTRY, int TRACKING>
-hipError_t launch_batch(const rtc8x_frame_params* d_params, const uint32_t* num_samples, const double* shares,
-                        uint32_t count, hipStream_t stream)
+// One persistent launch over several instances, a workgroup per CU; shares[i] is instance i's part of the
+// workgroups (each gets at least one), regions the largest region table.
+template <int ENTRY, int TRACKING, uint32_t REGION_BYTES>
+hipError_t launch_batch(const rtc8x_frame_params* params, const rtc8x_frame_params* d_params, const uint32_t* num_samples,
+                        const double* shares, uint32_t count, hipStream_t stream)
 {
-    const uint32_t slot = take_counter_slots();
-    int dev = 0, cus = 0, per_cu = 0;
+    const uint32_t ctr = take_counter_slots();
+    int dev = 0, cus = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (e != hipSuccess) return e;
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, batch_kernel<ENTRY, TRACKING>, 256, 0);
-    if (e != hipSuccess) return e;
-    if (per_cu < 1) per_cu = 1;
-    const uint32_t total = std::max<uint32_t>((uint32_t)(cus * per_cu), count);
+    const uint32_t total = std::max<uint32_t>((uint32_t)cus, count);
     BatchArgs b{};
     b.params = d_params;
     b.count = count;
-    b.slot = slot;
+    b.ctr = ctr;
     double sum = 0.0;
     for (uint32_t i = 0; i < count; ++i) sum += shares[i];
     uint32_t end = 0;
     double acc = 0.0;
+    bool few = true;
     for (uint32_t i = 0; i < count; ++i) {
         acc += shares[i];
         // cumulative rounding keeps the ranges summing to `total`; every instance keeps one workgroup
+        const uint32_t begin = end;
         uint32_t e_i = (uint32_t)std::llround(acc / sum * (total - count)) + i + 1;
         e_i = std::max(e_i, end + 1);
         b.wg_end[i] = end = std::min(e_i, total - (count - 1 - i));
         b.num_samples[i] = num_samples[i];
+        few &= few_paths((uint64_t)params[i].image_width * params[i].image_height, end - begin);
     }
-    hipLaunchKernelGGL(reset_counters_kernel, dim3(1), dim3(kMaxBatch), 0, stream, slot, count);
-    hipLaunchKernelGGL((batch_kernel<ENTRY, TRACKING>), dim3(end), dim3(256), 0, stream, b);
+    hipLaunchKernelGGL(reset_counters_kernel, dim3(1), dim3(kMaxBatch), 0, stream, ctr, count);
+    hipLaunchKernelGGL((slots_batch_kernel<ENTRY, TRACKING, REGION_BYTES, kSlotWaves>), dim3(end),
+                       dim3(64 * (few ? kSlotWavesFew : kSlotWaves)), 0, stream, b);
     return hipGetLastError();
+}
+
+template <int ENTRY>
+hipError_t launch_batch_tracking(const rtc8x_frame_params* params, const rtc8x_frame_params* d_params,
+                                 const uint32_t* num_samples, const double* shares, uint32_t count, hipStream_t stream)
+{
+    if (params[0].tracking != RTC8X_TRACKING_LOCAL_MAJORANT)
+        return launch_batch<ENTRY, RTC8X_TRACKING_GLOBAL_MAJORANT, 0>(params, d_params, num_samples, shares, count, stream);
+    uint32_t regions = 0;
+    for (uint32_t i = 0; i < count; ++i) regions = std::max(regions, region_bytes(params[i].grid));
+    if (regions <= kSmallRegions)
+        return launch_batch<ENTRY, RTC8X_TRACKING_LOCAL_MAJORANT, kSmallRegions>(params, d_params, num_samples, shares, count,
+                                                                                stream);
+    return launch_batch<ENTRY, RTC8X_TRACKING_LOCAL_MAJORANT, RTC8X_MAX_REGIONS>(params, d_params, num_samples, shares, count,
+                                                                                stream);
 }
 
 template <int ENTRY>
@@ -1773,21 +1765,6 @@ rtc8x_status check_batch(const char* who, const rtc8x_frame_params* params, cons
     return RTC8X_OK;
 }
 
-// The batched launch over a device copy `d` of the instances' frame parameters.
-hipError_t launch_batch_any(const rtc8x_frame_params* d, int32_t tracking, int32_t entry, const uint32_t* num_samples,
-                            const double* w, uint32_t count, hipStream_t s)
-{
-    if (tracking == RTC8X_TRACKING_LOCAL_MAJORANT)
-        return entry == RTC8X_ENTRY_PATH_TRACE
-                   ? dev::launch_batch<RTC8X_ENTRY_PATH_TRACE, RTC8X_TRACKING_LOCAL_MAJORANT>(d, num_samples, w, count, s)
-                   : dev::launch_batch<RTC8X_ENTRY_PATH_TRACE_WITH_NRC, RTC8X_TRACKING_LOCAL_MAJORANT>(d, num_samples, w,
-                                                                                                      count, s);
-    return entry == RTC8X_ENTRY_PATH_TRACE
-               ? dev::launch_batch<RTC8X_ENTRY_PATH_TRACE, RTC8X_TRACKING_GLOBAL_MAJORANT>(d, num_samples, w, count, s)
-               : dev::launch_batch<RTC8X_ENTRY_PATH_TRACE_WITH_NRC, RTC8X_TRACKING_GLOBAL_MAJORANT>(d, num_samples, w,
-                                                                                                   count, s);
-}
-
 }  // namespace
 
 namespace rtc8x {
@@ -1804,7 +1781,10 @@ rtc8x_status trace_batch_into(const char* who, void* stream, const rtc8x_frame_p
     RTC8X_REQUIRE(table != nullptr, "%s: no device table for the instances", who);
     hipStream_t s = (hipStream_t)stream;
     RTC8X_HIP(hipMemcpyAsync(table, params, sizeof(rtc8x_frame_params) * count, hipMemcpyHostToDevice, s));
-    RTC8X_HIP(launch_batch_any(table, params[0].tracking, entry, num_samples, w, count, s));
+    // over the device copy of the instances' frame parameters
+    RTC8X_HIP(entry == RTC8X_ENTRY_PATH_TRACE
+                  ? dev::launch_batch_tracking<RTC8X_ENTRY_PATH_TRACE>(params, table, num_samples, w, count, s)
+                  : dev::launch_batch_tracking<RTC8X_ENTRY_PATH_TRACE_WITH_NRC>(params, table, num_samples, w, count, s));
     return RTC8X_OK;
 }
 

@@ -162,3 +162,62 @@ def test_scheduling_knobs_do_not_change_results(entry):
         for a, b in zip(outs[0], o):
             assert np.array_equal(a, b)
     s.close()
+
+
+@pytest.mark.parametrize("tracking,region_cells", [(0, 0), (1, 0), (1, 2)])
+@pytest.mark.parametrize("shares", [None, [0.02, 1.0, 0.001, 0.3]])
+def test_counted_and_dealt_instances_in_one_batch(tracking, region_cells, shares):
+    """Instances whose pixels are dealt out, instances with more pixels than their workgroups hold (the work
+    counter, other workgroups helping) and one of a single pixel, by both entries; a small and a large region
+    table: the accumulators, PCG states, statistics and cache buffers of single launches, bit for bit."""
+    from rtcamp8_amd import _abi, batch
+    from rtcamp8_amd import scene as sc
+    from rtcamp8_amd._lib import call
+    from rtcamp8_amd.nrc import NrcRenderer
+    from rtcamp8_amd.tracer import PathTracer
+
+    base = _scenes()
+    sizes, spp = [(701, 547), (61, 43), (1, 1), (333, 97)], [2, 5, 7, 3]
+    cfgs = [base[i % 3].with_(width=w, height=h, tracking=tracking, env_kind="constant", max_path_length=48)
+            for i, (w, h) in enumerate(sizes)]
+    scenes = [sc.DeviceScene(c) for c in cfgs]
+    if region_cells:
+        for s in scenes:
+            call("rtc8x_grid_build_regions", C.byref(s.grid), region_cells)
+        assert max(int(np.prod(s.grid.region_dims[:])) for s in scenes) > 1000
+    tr = [[PathTracer(s) for s in scenes] for _ in range(2)]
+    for _ in range(2):  # the second launch in the work order of the first
+        for t, k in zip(tr[0], spp):
+            t.trace(k)
+        batch.trace_plain(tr[1], spp, shares)
+    for i, (a, b) in enumerate(zip(*tr)):
+        n = cfgs[i].width * cfgs[i].height
+        for x, y in ((a.accum, b.accum), (a.rng, b.rng), (a.stats, b.stats), (a.cost, b.cost)):
+            assert np.array_equal(x.download(np.uint32), y.download(np.uint32)), i
+        assert a.counters()["paths"] == 2 * n * spp[i]
+    for t in tr[0] + tr[1]:
+        t.close()
+    k = [2, 3, 1, 2]
+    keys = ("inference_queries", "inference_terminals", "per_frame_contribution")
+    got = []
+    for batched in (False, True):
+        rs = [NrcRenderer(s, samples_per_launch=3) for s in scenes]
+        for r in rs:
+            for key in keys:
+                getattr(r.buffers, key).fill(0)
+        ps = [r.params() for r in rs]
+        for p, kk in zip(ps, k):
+            p.nrc.num_samples = kk
+        if batched:
+            batch._launch(ps, k, _abi.ENTRY_PATH_TRACE_WITH_NRC, shares, None)
+        else:
+            for p, kk in zip(ps, k):
+                call("rtc8x_trace", None, C.byref(p), _abi.ENTRY_PATH_TRACE_WITH_NRC, kk)
+        got.append([[getattr(r.buffers, key).download(np.uint32) for key in keys] + [r.rng.download(np.uint32)] for r in rs])
+        for r in rs:
+            r.close()
+    for i, (a, b) in enumerate(zip(*got)):
+        for x, y in zip(a, b):
+            assert np.array_equal(x, y), i
+    for s in scenes:
+        s.close()
