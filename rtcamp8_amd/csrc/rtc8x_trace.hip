@@ -1,19 +1,17 @@
 // rtc8x_trace.hip -- the path-tracing launch: the three OptiX ray-generation programs
 // (pathTrace, generateTrainingData, pathTraceWithNRC; renderer/gpu_kernels/optix_pathtracing_kernels.cu
-// :31-448) for volume-only scenes.  The full-image launches run in rtc8x_slots.hpp; the training launch and
-// the batched launches run here, as one persistent per-lookup state machine.
+// :31-448) for volume-only scenes.  The full-image launches, single and batched, run in rtc8x_slots.hpp; the
+// training launch runs here, as one persistent per-lookup state machine.
 //
-// A lane owns one pixel at a time (all of its samples, so the pixel's PCG stream is consumed in the
-// reference's order) and steps its path through free-flight tracking towards the next scattering
+// A lane owns one pixel at a time and steps its path through free-flight tracking towards the next scattering
 // vertex, ratio tracking of the NEE shadow ray, and vertex events (camera ray, escape, scattering with
 // Russian roulette and NRC termination, NEE set-up, phase sampling, training records, path end).  Each
 // iteration of the main loop takes one tentative collision, with its density lookup, for every lane
 // that is stepping a segment; a lane that reaches a vertex event parks, and the parked lanes run their
-// events together once they are a quarter of the wavefront's active lanes, so that each event's code is
+// events together once they are 3/8 of the wavefront's active lanes, so that each event's code is
 // issued once for many lanes.  A lane whose pixel is done takes the next one from a work counter
-// (8x8 pixel tiles or a caller-given order, one atomic per wavefront).  Per pixel, the random numbers
-// and floating-point operations are the reference's, so results are bit-identical to tracing each
-// pixel's paths one after another.
+// (8x8 pixel tiles, one atomic per wavefront).  Per pixel, the random numbers and floating-point operations
+// are the reference's, so results are bit-identical to tracing each pixel's paths one after another.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -84,10 +82,10 @@ enum : uint32_t {
 };
 
 struct Lane {
-    uint32_t lx, ly, lin, sample, cost0, scat0;
+    uint32_t lx, ly, lin, cost0, scat0;
     Pcg rng;
     V3 org, dir, pos;
-    RGB tp, contribution, nee_f;
+    RGB tp, nee_f;
     float dir_pd, init_importance, vis, nee_k1, nee_k2, nee_k3;
     uint32_t path_length, mode;
     bool nee_sun;
@@ -432,63 +430,48 @@ __device__ __forceinline__ void train_dims(const rtc8x_frame_params& p, uint32_t
     th = (uint32_t)min(max(ts[1], 0), (int32_t)p.image_height);
 }
 
-// pathTrace_generic<withNRC, genData> (optix_pathtracing_kernels.cu:31-434) for volume-only scenes, as
-// a per-lookup state machine over a persistent grid.  ENTRY selects the ray-generation program;
-// GENERATE_TRAINING_DATA runs as the staging launch or the redo launch (TrainStage; the redo records at
-// record_offsets).
-template <int ENTRY, int TRACKING>
-__device__ __forceinline__ void trace_body(const rtc8x_frame_params& p, uint32_t launch_w, uint32_t launch_h,
-                                           uint32_t num_samples, uint32_t slot,
+// pathTrace_generic<withNRC, genData = true> (optix_pathtracing_kernels.cu:31-434) for volume-only scenes, as
+// a per-lookup state machine over a persistent grid: the staging launch or the redo launch (TrainStage; the
+// redo records at record_offsets).
+template <int TRACKING>
+__device__ __forceinline__ void trace_body(const rtc8x_frame_params& p, uint32_t slot,
                                            const uint32_t* __restrict__ record_offsets,
                                            uint32_t* __restrict__ record_counts, const TrainStage& stage,
                                            const uint8_t* __restrict__ region_table)
 {
-    constexpr bool with_nrc = ENTRY != RTC8X_ENTRY_PATH_TRACE;
-    constexpr bool gen_data = ENTRY == RTC8X_ENTRY_GENERATE_TRAINING_DATA;
     const rtc8x_nrc_buffers& nb = p.nrc;
-    const bool staged = gen_data && stage.counter != nullptr;
-    const bool redo = gen_data && stage.redo_lost != nullptr;
+    const bool staged = stage.counter != nullptr;
+    const bool redo = stage.redo_lost != nullptr;
     float* const train_targets = staged ? stage.targets : nb.train_targets[0];
-    // GENERATE_TRAINING_DATA is launched with a zero size and takes the training size from the device
-    uint32_t W = launch_w, H = launch_h;
-    if (gen_data && W == 0) train_dims(p, W, H);
+    uint32_t W, H;
+    train_dims(p, W, H);
     // pixel tiles of 64 lanes: 8x8, 16x4, 32x2 or 4x16
     const uint32_t tile_w = p.tile_shape == 1 ? 16u : (p.tile_shape == 2 ? 32u : (p.tile_shape == 3 ? 4u : 8u));
     const uint32_t tile_h = 64u / tile_w;
     const uint32_t tiles_x = (W + tile_w - 1) / tile_w;
-    // GENERATE_TRAINING_DATA hands out the unbiased-suffix pixels first (the one pixel of each 4x4 block
+    // The unbiased-suffix pixels are handed out first (the one pixel of each 4x4 block
     // with ((ly % 4) * 4 + lx % 4 + offset) % 16 == 0): their paths run to full length, so starting
     // them first keeps the launch from waiting on them at the end.
     const uint32_t first_c = (16u - nb.offset_to_select_unbiased_path % 16u) % 16u;
     const uint32_t first_rx = first_c % 4u, first_ry = first_c / 4u;
     const uint32_t first_nx = W > first_rx ? (W - first_rx + 3u) / 4u : 0u;
     const uint32_t first_ny = H > first_ry ? (H - first_ry + 3u) / 4u : 0u;
-    const uint32_t n_first = (gen_data && !p.work_order) ? first_nx * first_ny : 0u;
-    const uint32_t total = p.work_order ? W * H : n_first + tiles_x * ((H + tile_h - 1) / tile_h) * 64;
+    const uint32_t n_first = first_nx * first_ny;
+    const uint32_t total = n_first + tiles_x * ((H + tile_h - 1) / tile_h) * 64;
     // A training launch with few paths for the persistent grid (frame 0's quarter-size training image,
     // a small frame) is bound by its longest paths' chains of lookups, not by throughput.  Its
     // wavefronts then take at most `lanes` paths each, so that the paths spread over the whole grid and
     // every wavefront has the idle lanes that take its paths' segments cooperatively from the start.
     uint32_t lanes = 64;
-    if constexpr (gen_data) {
+    {
         const uint32_t waves = gridDim.x * (blockDim.x >> 6);
         const uint32_t per = (total + waves - 1) / waves;
         if (per <= kTrainSpreadLanes) lanes = per > 0 ? per : 1u;
     }
-    // default event thresholds, measured on the 512^3 cloud at 1080p: the render entries 5/8 with the
-    // local walk (4/8 gave 35.1 against 34.7 ms per plain 16-spp frame, 6/8 34.7) and 4/8 with the global
-    // one (3/8: 44.0 against 43.2 ms); the training entry 3/8 (no difference measured)
-    constexpr uint32_t kEv8Default = ENTRY == RTC8X_ENTRY_GENERATE_TRAINING_DATA     ? 3u
-                                     : TRACKING == RTC8X_TRACKING_LOCAL_MAJORANT ? 5u
-                                                                                 : 4u;
-    const uint32_t ev8 = (p.event_eighths >= 1 && p.event_eighths <= 8) ? p.event_eighths : kEv8Default;
+    // the default event threshold (2/8 to 5/8: no difference measured)
+    const uint32_t ev8 = (p.event_eighths >= 1 && p.event_eighths <= 8) ? p.event_eighths : 3u;
     const uint32_t lane_id = threadIdx.x & 63;
-    // per-sample slices of the render buffers (one launch may trace several samples into the cache)
-    const size_t q_stride = ((size_t)W * H + 127u) & ~(size_t)127u, p_stride = (size_t)W * H;
-    uint32_t max_len = (ENTRY == RTC8X_ENTRY_PATH_TRACE && p.max_path_length) ? p.max_path_length : kHardMaxPathLength;
-    if (max_len > kHardMaxPathLength) max_len = kHardMaxPathLength;
-    uint32_t rr_after = p.rr_after_path_length;
-    if (gen_data && rr_after < 2) rr_after = 2;
+    const uint32_t rr_after = p.rr_after_path_length < 2 ? 2u : p.rr_after_path_length;
     const float prob_env = (p.sun.enabled && p.env.kind != RTC8X_ENV_NONE) ? 1.0f - p.sun.select_prob : 1.0f;
 
     Medium med;
@@ -503,28 +486,21 @@ __device__ __forceinline__ void trace_body(const rtc8x_frame_params& p, uint32_t
     for (;;) {
         // Vertex events are batched: a lane that reaches one parks, and once enough of the wavefront's
         // active lanes have parked they run their events together (each event block is issued once for
-        // many lanes instead of once per lane), while the others keep stepping through lookups.  The
-        // plain and training entries then run only the larger of the two vertex events (a real
+        // many lanes instead of once per lane), while the others keep stepping through lookups.  From
+        // event_eighths / 8 of the active lanes on, only the larger of the two vertex events (a real
         // collision: Russian roulette and NEE set-up; an NEE segment's end: phase sampling and the next
-        // segment) together with the path starts and ends, from event_eighths / 8 of the active lanes;
-        // the other event's lanes wait for a later pass.  The NRC render entry, whose paths are short,
-        // runs every parked lane from event_eighths / 8.
+        // segment) runs, together with the path starts and ends; the other event's lanes wait for a later
+        // pass.
         const uint64_t parked = __ballot(L.mode != kModeTrack && L.mode != kModeShadow && L.mode != kModeIdle);
         const uint64_t stepping = __ballot(L.mode == kModeTrack || L.mode == kModeShadow);
         if (parked == 0 && stepping == 0) break;
         const uint32_t n_parked = __popcll(parked), n_active = __popcll(parked | stepping);
-        bool run_events;
-        if constexpr (ENTRY == RTC8X_ENTRY_PATH_TRACE_WITH_NRC) {
-            run_events = stepping == 0 || 8 * n_parked >= ev8 * n_active;
-        } else {
-            run_events = stepping == 0;
-            if (!run_events && 8 * n_parked >= ev8 * n_active) {
-                const uint64_t at_collision = __ballot(L.mode == kModeScatter), at_nee_end = __ballot(L.mode == kModeNeeDone);
-                const uint64_t others = parked & ~(at_collision | at_nee_end);
-                const uint64_t sel =
-                    (__popcll(at_collision) >= __popcll(at_nee_end) ? at_collision : at_nee_end) | others;
-                run_events = ((sel >> lane_id) & 1ull) != 0;
-            }
+        bool run_events = stepping == 0;
+        if (!run_events && 8 * n_parked >= ev8 * n_active) {
+            const uint64_t at_collision = __ballot(L.mode == kModeScatter), at_nee_end = __ballot(L.mode == kModeNeeDone);
+            const uint64_t others = parked & ~(at_collision | at_nee_end);
+            const uint64_t sel = (__popcll(at_collision) >= __popcll(at_nee_end) ? at_collision : at_nee_end) | others;
+            run_events = ((sel >> lane_id) & 1ull) != 0;
         }
         // ---- events until this lane has a tracking or shadow segment under way, or no work left
         while (run_events && L.mode != kModeIdle && L.mode != kModeTrack && L.mode != kModeShadow) {
@@ -544,29 +520,23 @@ __device__ __forceinline__ void trace_body(const rtc8x_frame_params& p, uint32_t
                     L.mode = kModeIdle;
                     continue;
                 }
-                if (p.work_order) {
-                    const uint32_t lin = p.work_order[w];
-                    if (lin >= W * H) continue;
-                    L.lx = lin % W;
-                    L.ly = lin / W;
-                } else if (gen_data && w < n_first) {
+                if (w < n_first) {
                     L.lx = 4 * (w % first_nx) + first_rx;
                     L.ly = 4 * (w / first_nx) + first_ry;
                 } else {
-                    const uint32_t wt = gen_data ? w - n_first : w;
+                    const uint32_t wt = w - n_first;
                     const uint32_t tile = wt >> 6, within = wt & 63u;
                     L.lx = (tile % tiles_x) * tile_w + within % tile_w;
                     L.ly = (tile / tiles_x) * tile_h + within / tile_w;
                     if (L.lx >= W || L.ly >= H) continue;
-                    if (gen_data && (L.lx & 3u) == first_rx && (L.ly & 3u) == first_ry) continue;  // taken first
+                    if ((L.lx & 3u) == first_rx && (L.ly & 3u) == first_ry) continue;  // taken first
                 }
                 L.lin = L.ly * W + L.lx;
                 if (redo && !stage.redo_lost[L.lin]) continue;  // all of its records were staged
                 L.cost0 = med.lookups;
                 L.scat0 = scatters;
                 L.rng.state = redo ? stage.rng_save[L.lin] : p.rng_states[(size_t)L.ly * p.image_width + L.lx];
-                L.sample = 0;
-                if (gen_data) L.train_base = record_offsets ? record_offsets[L.lin] : 0u;
+                L.train_base = record_offsets ? record_offsets[L.lin] : 0u;
                 L.mode = kModeStart;
             }
             if (L.mode == kModeStart) {
@@ -582,23 +552,18 @@ __device__ __forceinline__ void trace_body(const rtc8x_frame_params& p, uint32_t
                 L.dir = normalize(dir);
                 float az = ldir.z < 0.0f ? -ldir.z : ldir.z;
                 L.dir_pd = 1.0f / (az * (az * az) * sensor_area);
-                L.contribution = RGB{0.0f, 0.0f, 0.0f};
                 float rinv = 1.0f / L.dir_pd;
                 L.tp = RGB{rinv, rinv, rinv};
                 L.init_importance = luminance(L.tp);
                 L.path_length = 1;
-                if (with_nrc) {
-                    L.primary_spread = 0.0f;
-                    L.cur_sqrt_spread = 0.0f;
-                }
-                if (gen_data) {
-                    const uint32_t tl = (L.ly % 4u) * 4u + (L.lx % 4u);
-                    L.unbiased = ((tl + nb.offset_to_select_unbiased_path) % 16u) == 0;
-                    L.prev_idx = RTC8X_INVALID_VERTEX_INDEX;
-                    L.prev_local_tp = RGB{0.0f, 0.0f, 0.0f};
-                    L.records = 0;
-                    L.lost = false;
-                }
+                L.primary_spread = 0.0f;
+                L.cur_sqrt_spread = 0.0f;
+                const uint32_t tl = (L.ly % 4u) * 4u + (L.lx % 4u);
+                L.unbiased = ((tl + nb.offset_to_select_unbiased_path) % 16u) == 0;
+                L.prev_idx = RTC8X_INVALID_VERTEX_INDEX;
+                L.prev_local_tp = RGB{0.0f, 0.0f, 0.0f};
+                L.records = 0;
+                L.lost = false;
                 L.mode = start_segment<TRACKING>(p.grid, med, sg, L.rng, L.org, L.dir, 1e10f) ? kModeTrack : kModeEscape;
             }
             bool after_nee = false, path_end = false;
@@ -614,8 +579,7 @@ __device__ __forceinline__ void trace_body(const rtc8x_frame_params& p, uint32_t
                         mis = bsdf_pd * bsdf_pd / (bsdf_pd * bsdf_pd + light_pd * light_pd);
                     }
                     const RGB implicit_cont = scale(radiance, mis);
-                    if (!gen_data) L.contribution = add(L.contribution, mul(L.tp, implicit_cont));
-                    if (gen_data && L.prev_idx != RTC8X_INVALID_VERTEX_INDEX) {
+                    if (L.prev_idx != RTC8X_INVALID_VERTEX_INDEX) {
                         float* tgt = train_targets + 3 * (size_t)L.prev_idx;
                         const RGB a = mul(L.prev_local_tp, implicit_cont);
                         tgt[0] = tgt[0] + a.r;
@@ -623,21 +587,12 @@ __device__ __forceinline__ void trace_body(const rtc8x_frame_params& p, uint32_t
                         tgt[2] = tgt[2] + a.b;
                     }
                 }
-                if (gen_data) {
-                    rtc8x_training_suffix_terminal ti;
-                    ti.prev_vertex_index = L.prev_idx;
-                    ti.has_query = 0;
-                    ti.path_length = L.path_length & 0xFFu;
-                    ti.is_unbiased = L.unbiased ? 1u : 0u;
-                    nb.train_suffix_terminals[L.lin] = ti;
-                } else if (with_nrc) {
-                    rtc8x_terminal_info ti;
-                    ti.throughput[0] = L.tp.r;
-                    ti.throughput[1] = L.tp.g;
-                    ti.throughput[2] = L.tp.b;
-                    ti.has_query = (L.path_length & 0xFFu) << 8;
-                    nb.inference_terminals[(size_t)L.sample * p_stride + L.lin] = ti;
-                }
+                rtc8x_training_suffix_terminal ti;
+                ti.prev_vertex_index = L.prev_idx;
+                ti.has_query = 0;
+                ti.path_length = L.path_length & 0xFFu;
+                ti.is_unbiased = L.unbiased ? 1u : 0u;
+                nb.train_suffix_terminals[L.lin] = ti;
                 path_end = true;
             } else if (L.mode == kModeNeeDone) {
                 // end of the NEE shadow ray (performNextEventEstimation, renderer_kernel_common.h:297-403)
@@ -645,23 +600,20 @@ __device__ __forceinline__ void trace_body(const rtc8x_frame_params& p, uint32_t
                 if (L.vis > 0.0f)
                     nee_c = L.nee_sun ? scale(L.nee_f, L.vis / L.nee_k1)
                                       : scale(L.nee_f, L.vis * L.nee_k1 * L.nee_k2 / L.nee_k3);
-                if (!gen_data) L.contribution = add(L.contribution, mul(L.tp, nee_c));
-                if (gen_data) L.nee_c = nee_c;
+                L.nee_c = nee_c;
                 after_nee = true;
             } else if (L.mode == kModeScatter) {
                 // medium interaction at sg.t (optix_pathtracing_kernels.cu:176-268)
                 scatters++;
                 const float th = sg.t;
                 L.pos = V3{L.org.x + th * L.dir.x, L.org.y + th * L.dir.y, L.org.z + th * L.dir.z};
-                if (with_nrc) {
-                    // path spread (optix_pathtracing_kernels.cu:200-210)
-                    float ddx = L.pos.x - L.org.x, ddy = L.pos.y - L.org.y, ddz = L.pos.z - L.org.z;
-                    float dist2 = ddx * ddx + ddy * ddy + ddz * ddz;
-                    if (L.path_length == 1)
-                        L.primary_spread = dist2 / (4.0f * RTC8X_PI_F * 1.0f);
-                    else
-                        L.cur_sqrt_spread += sqrtf(dist2 / (L.dir_pd * 1.0f));
-                }
+                // path spread (optix_pathtracing_kernels.cu:200-210)
+                float ddx = L.pos.x - L.org.x, ddy = L.pos.y - L.org.y, ddz = L.pos.z - L.org.z;
+                float dist2 = ddx * ddx + ddy * ddy + ddz * ddz;
+                if (L.path_length == 1)
+                    L.primary_spread = dist2 / (4.0f * RTC8X_PI_F * 1.0f);
+                else
+                    L.cur_sqrt_spread += sqrtf(dist2 / (L.dir_pd * 1.0f));
                 // Russian roulette (optix_pathtracing_kernels.cu:254-268)
                 float continue_prob = 1.0f;
                 bool rr_terminated = false;
@@ -670,37 +622,20 @@ __device__ __forceinline__ void trace_body(const rtc8x_frame_params& p, uint32_t
                     continue_prob = fminf(q, 1.0f);
                     if (L.rng.uni() >= continue_prob) rr_terminated = true;
                 }
-                if (!with_nrc && rr_terminated) path_end = true;
-                if (with_nrc) {
-                    // termination into the cache (optix_pathtracing_kernels.cu:282-330)
-                    bool ends_with_cache = rr_terminated;
-                    const float pt = nb.path_termination_factor;
-                    if (gen_data) {
-                        if (!L.unbiased)
-                            ends_with_cache |= L.cur_sqrt_spread * L.cur_sqrt_spread > 2.0f * pt * L.primary_spread;
-                    } else {
-                        ends_with_cache |= L.cur_sqrt_spread * L.cur_sqrt_spread > pt * L.primary_spread;
-                    }
-                    if (ends_with_cache) {
-                        const V3 vout{-L.dir.x, -L.dir.y, -L.dir.z};
-                        make_query(p, L.pos, vout, &nb.inference_queries[(size_t)L.sample * q_stride + L.lin]);
-                        if (gen_data) {
-                            rtc8x_training_suffix_terminal ti;
-                            ti.prev_vertex_index = L.prev_idx;
-                            ti.has_query = 1;
-                            ti.path_length = L.path_length & 0xFFu;
-                            ti.is_unbiased = L.unbiased ? 1u : 0u;
-                            nb.train_suffix_terminals[L.lin] = ti;
-                        } else {
-                            rtc8x_terminal_info ti;
-                            ti.throughput[0] = L.tp.r;
-                            ti.throughput[1] = L.tp.g;
-                            ti.throughput[2] = L.tp.b;
-                            ti.has_query = 1u | ((L.path_length & 0xFFu) << 8);
-                            nb.inference_terminals[(size_t)L.sample * p_stride + L.lin] = ti;
-                        }
-                        path_end = true;
-                    }
+                // termination into the cache (optix_pathtracing_kernels.cu:282-330)
+                bool ends_with_cache = rr_terminated;
+                const float pt = nb.path_termination_factor;
+                if (!L.unbiased)
+                    ends_with_cache |= L.cur_sqrt_spread * L.cur_sqrt_spread > 2.0f * pt * L.primary_spread;
+                if (ends_with_cache) {
+                    make_query(p, L.pos, V3{-L.dir.x, -L.dir.y, -L.dir.z}, &nb.inference_queries[L.lin]);
+                    rtc8x_training_suffix_terminal ti;
+                    ti.prev_vertex_index = L.prev_idx;
+                    ti.has_query = 1;
+                    ti.path_length = L.path_length & 0xFFu;
+                    ti.is_unbiased = L.unbiased ? 1u : 0u;
+                    nb.train_suffix_terminals[L.lin] = ti;
+                    path_end = true;
                 }
                 if (!path_end) {
                     L.tp = scale(L.tp, 1.0f / continue_prob);
@@ -748,9 +683,7 @@ __device__ __forceinline__ void trace_body(const rtc8x_frame_params& p, uint32_t
                         if (lp_cos <= 0.0f) zero = true;
                     }
                     if (zero) {
-                        const RGB nee_c{0.0f, 0.0f, 0.0f};
-                        if (!gen_data) L.contribution = add(L.contribution, mul(L.tp, nee_c));
-                        if (gen_data) L.nee_c = nee_c;
+                        L.nee_c = RGB{0.0f, 0.0f, 0.0f};
                         after_nee = true;
                     } else {
                         const Frame fr = make_frame(V3{-L.dir.x, -L.dir.y, -L.dir.z});
@@ -782,7 +715,7 @@ __device__ __forceinline__ void trace_body(const rtc8x_frame_params& p, uint32_t
                 }
             }
             if (after_nee) {
-                if (L.path_length >= max_len) {
+                if (L.path_length >= kHardMaxPathLength) {
                     path_end = true;
                 } else {
                     // phase sampling (optix_pathtracing_kernels.cu:341-356)
@@ -803,57 +736,55 @@ __device__ __forceinline__ void trace_body(const rtc8x_frame_params& p, uint32_t
                         L.org = L.pos;
                         L.dir_pd = pdf;
                         bool record_end = false;
-                        if (gen_data) {
-                            // training vertex record (optix_pathtracing_kernels.cu:358-410)
-                            const uint32_t local = L.records;
-                            L.records++;
-                            rtc8x_radiance_query q;
-                            make_query(p, L.pos, vout, &q);
-                            // the record's slot: the next staging slot, or in pixel order (redo launch)
-                            const uint32_t idx = staged ? atomicAdd(stage.counter, 1u) : L.train_base + local;
-                            if (staged && idx >= kStageCapacity) {
-                                // no staging slot left: the redo launch traces this pixel again
-                                L.prev_idx = RTC8X_INVALID_VERTEX_INDEX;
-                                L.lost = true;
-                            } else if (staged || idx < RTC8X_TRAIN_BUFFER_SIZE) {
-                                (staged ? stage.queries : nb.train_queries[0])[idx] = q;
-                                rtc8x_training_vertex_info vi;
-                                vi.local_throughput[0] = local_tp.r;
-                                vi.local_throughput[1] = local_tp.g;
-                                vi.local_throughput[2] = local_tp.b;
-                                vi.prev_vertex_index = L.prev_idx;
-                                vi.path_length = L.path_length & 0xFFu;
-                                vi.is_unbiased = L.unbiased ? 1u : 0u;
-                                if (staged) {
-                                    stage.info[idx] = vi;
-                                    stage.tag[2 * (size_t)idx] = L.lin;
-                                    stage.tag[2 * (size_t)idx + 1] = local;
-                                    StageSnapshot sn;
-                                    sn.rng = L.rng.state;
-                                    sn.path_length = L.path_length;
-                                    sn.lookups = med.lookups - L.cost0;
-                                    sn.scatters = scatters - L.scat0;
-                                    sn.pad = 0;
-                                    stage.snap[idx] = sn;
-                                } else {
-                                    nb.train_vertex_info[idx] = vi;
-                                }
-                                float* tgt = train_targets + 3 * (size_t)idx;
-                                tgt[0] = L.nee_c.r;
-                                tgt[1] = L.nee_c.g;
-                                tgt[2] = L.nee_c.b;
-                                L.prev_local_tp = local_tp;
-                                L.prev_idx = idx;
+                        // training vertex record (optix_pathtracing_kernels.cu:358-410)
+                        const uint32_t local = L.records;
+                        L.records++;
+                        rtc8x_radiance_query q;
+                        make_query(p, L.pos, vout, &q);
+                        // the record's slot: the next staging slot, or in pixel order (redo launch)
+                        const uint32_t idx = staged ? atomicAdd(stage.counter, 1u) : L.train_base + local;
+                        if (staged && idx >= kStageCapacity) {
+                            // no staging slot left: the redo launch traces this pixel again
+                            L.prev_idx = RTC8X_INVALID_VERTEX_INDEX;
+                            L.lost = true;
+                        } else if (staged || idx < RTC8X_TRAIN_BUFFER_SIZE) {
+                            (staged ? stage.queries : nb.train_queries[0])[idx] = q;
+                            rtc8x_training_vertex_info vi;
+                            vi.local_throughput[0] = local_tp.r;
+                            vi.local_throughput[1] = local_tp.g;
+                            vi.local_throughput[2] = local_tp.b;
+                            vi.prev_vertex_index = L.prev_idx;
+                            vi.path_length = L.path_length & 0xFFu;
+                            vi.is_unbiased = L.unbiased ? 1u : 0u;
+                            if (staged) {
+                                stage.info[idx] = vi;
+                                stage.tag[2 * (size_t)idx] = L.lin;
+                                stage.tag[2 * (size_t)idx + 1] = local;
+                                StageSnapshot sn;
+                                sn.rng = L.rng.state;
+                                sn.path_length = L.path_length;
+                                sn.lookups = med.lookups - L.cost0;
+                                sn.scatters = scatters - L.scat0;
+                                sn.pad = 0;
+                                stage.snap[idx] = sn;
                             } else {
-                                nb.inference_queries[L.lin] = q;
-                                rtc8x_training_suffix_terminal ti;
-                                ti.prev_vertex_index = L.prev_idx;
-                                ti.has_query = 1;
-                                ti.path_length = L.path_length & 0xFFu;
-                                ti.is_unbiased = L.unbiased ? 1u : 0u;
-                                nb.train_suffix_terminals[L.lin] = ti;
-                                record_end = true;
+                                nb.train_vertex_info[idx] = vi;
                             }
+                            float* tgt = train_targets + 3 * (size_t)idx;
+                            tgt[0] = L.nee_c.r;
+                            tgt[1] = L.nee_c.g;
+                            tgt[2] = L.nee_c.b;
+                            L.prev_local_tp = local_tp;
+                            L.prev_idx = idx;
+                        } else {
+                            nb.inference_queries[L.lin] = q;
+                            rtc8x_training_suffix_terminal ti;
+                            ti.prev_vertex_index = L.prev_idx;
+                            ti.has_query = 1;
+                            ti.path_length = L.path_length & 0xFFu;
+                            ti.is_unbiased = L.unbiased ? 1u : 0u;
+                            nb.train_suffix_terminals[L.lin] = ti;
+                            record_end = true;
                         }
                         if (record_end) {
                             path_end = true;
@@ -876,28 +807,9 @@ __device__ __forceinline__ void trace_body(const rtc8x_frame_params& p, uint32_t
                     stage.scatters[L.lin] = scatters - L.scat0;
                     stage.lost[L.lin] = L.lost ? 1u : 0u;
                 }
-                const bool ok = all_nonneg_finite(L.contribution);
-                if (ENTRY == RTC8X_ENTRY_PATH_TRACE) {
-                    if (ok) {
-                        double* a = p.accum + 3 * (size_t)L.lin;
-                        a[0] += (double)L.contribution.r;
-                        a[1] += (double)L.contribution.g;
-                        a[2] += (double)L.contribution.b;
-                    }
-                } else if (ENTRY == RTC8X_ENTRY_PATH_TRACE_WITH_NRC) {
-                    float* pf = nb.per_frame_contribution + 3 * ((size_t)L.sample * p_stride + L.lin);
-                    pf[0] = ok ? L.contribution.r : 0.0f;
-                    pf[1] = ok ? L.contribution.g : 0.0f;
-                    pf[2] = ok ? L.contribution.b : 0.0f;
-                }
                 if (p.path_vertices && !staged) p.path_vertices[L.lin] += L.path_length;
-                if (++L.sample < num_samples) {
-                    L.mode = kModeStart;
-                } else {
-                    p.rng_states[(size_t)L.ly * p.image_width + L.lx] = L.rng.state;
-                    if (p.pixel_cost) p.pixel_cost[L.lin] = med.lookups - L.cost0;
-                    L.mode = kModeWork;
-                }
+                p.rng_states[(size_t)L.ly * p.image_width + L.lx] = L.rng.state;
+                L.mode = kModeWork;
             }
         }
         // ---- tentative collisions, with their density lookups, for every stepping lane
@@ -906,7 +818,7 @@ __device__ __forceinline__ void trace_body(const rtc8x_frame_params& p, uint32_t
             const uint64_t steppers = __ballot(L.mode == kModeTrack || L.mode == kModeShadow);
             coop = steppers != 0 && __popcll(__ballot(L.mode == kModeIdle)) >= kCoopIdle;
             if (coop) coop_segments(p.grid, med, sg, L, steppers, lane_id);
-        } else if constexpr (ENTRY == RTC8X_ENTRY_GENERATE_TRAINING_DATA) {
+        } else {
             // a local path's 64 collisions cost one walk over their regions (tens of microseconds), while
             // the stepping lanes walk side by side: only the last few paths are taken this way
             const uint64_t steppers = __ballot(L.mode == kModeTrack || L.mode == kModeShadow);
@@ -917,7 +829,7 @@ __device__ __forceinline__ void trace_body(const rtc8x_frame_params& p, uint32_t
         if (coop) {
         } else if constexpr (TRACKING == RTC8X_TRACKING_GLOBAL_MAJORANT) {
             // one copy of the lookup code serves both segment kinds: the kernel's instruction footprint
-            // matters (a copy per kind made the full-image launch half again as slow)
+            // matters (a copy per kind made a launch half again as slow)
             if (L.mode == kModeTrack || L.mode == kModeShadow)
                 speculate_global<kSpeculate>(p.grid, med, sg, L, L.mode == kModeTrack);
         } else if (L.mode == kModeTrack || L.mode == kModeShadow) {
@@ -1001,23 +913,15 @@ inline uint32_t take_counter_slots()
     return (next.fetch_add(1) % (kCounterSlots / kMaxBatch)) * kMaxBatch;
 }
 
-// One launch of one image.
-// Local tracking keeps a region walk per lane on top of the lane state: the render entries are held to
-// three wavefronts per SIMD (168 VGPRs, a few spilled); the training entry, whose lane state is larger,
-// would spill too much and keeps its registers.
-template <int ENTRY, int TRACKING>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
-    TRACKING == RTC8X_TRACKING_LOCAL_MAJORANT && ENTRY != RTC8X_ENTRY_GENERATE_TRAINING_DATA ? 3 : 1)))
-void wavefront_kernel(const rtc8x_frame_params p, uint32_t launch_w,
-                                                        uint32_t launch_h, uint32_t num_samples, uint32_t slot,
+// The training launch (staging or redo).
+template <int TRACKING>
+__global__ __launch_bounds__(256) void wavefront_kernel(const rtc8x_frame_params p, uint32_t slot,
                                                         const uint32_t* __restrict__ record_offsets,
                                                         uint32_t* __restrict__ record_counts, const TrainStage stage)
 {
-    if constexpr (ENTRY == RTC8X_ENTRY_GENERATE_TRAINING_DATA) {
-        // every record found a staging slot: no pixel for the redo launch (a walk over the training image
-        // that skips every pixel took about 0.1 ms)
-        if (stage.redo_lost != nullptr && *stage.staged <= kStageCapacity) return;
-    }
+    // every record found a staging slot: no pixel for the redo launch (a walk over the training image that
+    // skips every pixel took about 0.1 ms)
+    if (stage.redo_lost != nullptr && *stage.staged <= kStageCapacity) return;
     if constexpr (TRACKING == RTC8X_TRACKING_LOCAL_MAJORANT) {
         // the region majorants staged in LDS: every DDA step reads them there
         __shared__ __align__(16) uint8_t regions[RTC8X_MAX_REGIONS];
@@ -1026,11 +930,9 @@ void wavefront_kernel(const rtc8x_frame_params p, uint32_t launch_w,
         const uint4* src = reinterpret_cast<const uint4*>(p.grid.region_majorants);
         for (uint32_t i = threadIdx.x; i < n16; i += blockDim.x) reinterpret_cast<uint4*>(regions)[i] = src[i];
         __syncthreads();
-        trace_body<ENTRY, TRACKING>(p, launch_w, launch_h, num_samples, slot, record_offsets, record_counts, stage,
-                                    regions);
+        trace_body<TRACKING>(p, slot, record_offsets, record_counts, stage, regions);
     } else {
-        trace_body<ENTRY, TRACKING>(p, launch_w, launch_h, num_samples, slot, record_offsets, record_counts, stage,
-                                    nullptr);
+        trace_body<TRACKING>(p, slot, record_offsets, record_counts, stage, nullptr);
     }
 }
 
@@ -1379,9 +1281,9 @@ __global__ __launch_bounds__(256) void tile_expand_kernel(const uint32_t* __rest
 // One persistent launch: as many 256-lane workgroups as fit on the device at once, a fresh work
 // counter slot (cleared by a one-lane kernel on the same stream; launches on different streams take
 // different slots).
-template <int ENTRY, int TRACKING>
-hipError_t launch(const rtc8x_frame_params& p, uint32_t w, uint32_t h, uint32_t num_samples, const uint32_t* offsets,
-                  uint32_t* counts, const TrainStage& stage, hipStream_t stream)
+template <int TRACKING>
+hipError_t launch(const rtc8x_frame_params& p, const uint32_t* offsets, uint32_t* counts, const TrainStage& stage,
+                  hipStream_t stream)
 {
     const uint32_t slot = take_counter_slots();
     int dev = 0, cus = 0, per_cu = 0;
@@ -1389,12 +1291,12 @@ hipError_t launch(const rtc8x_frame_params& p, uint32_t w, uint32_t h, uint32_t 
     if (e != hipSuccess) return e;
     e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (e != hipSuccess) return e;
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wavefront_kernel<ENTRY, TRACKING>, 256, 0);
+    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wavefront_kernel<TRACKING>, 256, 0);
     if (e != hipSuccess) return e;
     if (per_cu < 1) per_cu = 1;
     hipLaunchKernelGGL(reset_counter_kernel, dim3(1), dim3(1), 0, stream, slot);
-    hipLaunchKernelGGL((wavefront_kernel<ENTRY, TRACKING>), dim3((uint32_t)(cus * per_cu)), dim3(256), 0,
-                       stream, p, w, h, num_samples, slot, offsets, counts, stage);
+    hipLaunchKernelGGL((wavefront_kernel<TRACKING>), dim3((uint32_t)(cus * per_cu)), dim3(256), 0, stream, p, slot, offsets,
+                       counts, stage);
     return hipGetLastError();
 }
 
@@ -1489,13 +1391,12 @@ hipError_t launch_batch_tracking(const rtc8x_frame_params* params, const rtc8x_f
                                                                                 stream);
 }
 
-template <int ENTRY>
-hipError_t launch_tracking(const rtc8x_frame_params& p, uint32_t w, uint32_t h, uint32_t ns, const uint32_t* offsets,
-                           uint32_t* counts, hipStream_t stream, const TrainStage& stage = TrainStage{})
+hipError_t launch_training(const rtc8x_frame_params& p, const uint32_t* offsets, uint32_t* counts,
+                           const TrainStage& stage, hipStream_t stream)
 {
     if (p.tracking == RTC8X_TRACKING_LOCAL_MAJORANT)
-        return launch<ENTRY, RTC8X_TRACKING_LOCAL_MAJORANT>(p, w, h, ns, offsets, counts, stage, stream);
-    return launch<ENTRY, RTC8X_TRACKING_GLOBAL_MAJORANT>(p, w, h, ns, offsets, counts, stage, stream);
+        return launch<RTC8X_TRACKING_LOCAL_MAJORANT>(p, offsets, counts, stage, stream);
+    return launch<RTC8X_TRACKING_GLOBAL_MAJORANT>(p, offsets, counts, stage, stream);
 }
 
 }  // namespace dev
@@ -1633,7 +1534,7 @@ rtc8x_status check_launch(const rtc8x_frame_params& p, int32_t entry, uint32_t n
                           "rtc8x_trace: local-majorant tracking needs region majorants");
     }
     if (p.tracking == RTC8X_TRACKING_LOCAL_MAJORANT) {
-        // the single-image kernel stages the whole region table in LDS
+        // the kernels stage the whole region table in LDS
         const int64_t nr = (int64_t)std::max(g.region_dims[0], 0) * std::max(g.region_dims[1], 0) *
                            std::max(g.region_dims[2], 0);
         RTC8X_REQUIRE(nr <= RTC8X_MAX_REGIONS && (nr == 0 || g.region_majorants),
@@ -1715,7 +1616,7 @@ try {
     stage.lost = reinterpret_cast<uint32_t*>(sb + lay.lost);
     hipLaunchKernelGGL(dev::reset_value_kernel, dim3(1), dim3(1), 0, s, stage.counter);
     RTC8X_HIP(hipGetLastError());
-    RTC8X_HIP((dev::launch_tracking<RTC8X_ENTRY_GENERATE_TRAINING_DATA>(p, 0, 0, 1, nullptr, counts, s, stage)));
+    RTC8X_HIP(dev::launch_training(p, nullptr, counts, stage, s));
     {
         // the training image is at most the frame's image: tiles over that bound, the extra ones exit
         const uint32_t tiles = (uint32_t)(((size_t)p.image_width * p.image_height + kPrefixTile - 1) / kPrefixTile);
@@ -1733,7 +1634,7 @@ try {
     redo.redo_lost = stage.lost;
     redo.rng_save = rng_save;
     redo.staged = stage.counter;
-    RTC8X_HIP((dev::launch_tracking<RTC8X_ENTRY_GENERATE_TRAINING_DATA>(p, 0, 0, 1, offsets, nullptr, s, redo)));
+    RTC8X_HIP(dev::launch_training(p, offsets, nullptr, redo, s));
     return RTC8X_OK;
 }
 RTC8X_CATCH_ALL("rtc8x_trace")
