@@ -411,12 +411,14 @@ struct Medium {
         normal = majorant >= 0x1p-40f && majorant <= 0x1p40f &&
                  (!g.region_majorants || (unit >= 0x1p-40f && unit <= 0x1p33f));
     }
-    // a over a majorant.  Voxels may be infinite or as large as floats are, whatever the majorants: those are
-    // divided in full, and no others (the fast division makes a NaN of infinity).
-    __device__ __forceinline__ float over(float a, float mu) const
+    // A density over a majorant.  Voxels may be infinite or as large as floats are, whatever the majorants: those
+    // are divided in full, and no others (the fast division makes a NaN of infinity).
+    __device__ __forceinline__ float over(float sigma, float mu) const
     {
-        return normal && fabsf(a) <= 0x1p40f ? div_normal(a, mu) : a / mu;
+        return normal && fabsf(sigma) <= 0x1p40f ? div_normal(sigma, mu) : sigma / mu;
     }
+    // An optical depth (at most 16) over a majorant: a distance.
+    __device__ __forceinline__ float distance(float tau, float mu) const { return normal ? div_normal(tau, mu) : tau / mu; }
 };
 
 // Density coefficient times the trilinear grid value at o + t d (no lookup counting).
@@ -643,7 +645,7 @@ struct Seg<RTC8X_TRACKING_LOCAL_MAJORANT> {
             if (res != kAdvanceBudget) break;
         }
         if (res == kAdvanceCollision) {
-            t = t + m.over(tau, mu_r);
+            t = t + m.distance(tau, mu_r);
             mu = mu_r;
         }
         return res;

@@ -186,8 +186,8 @@ void march_probe_kernel(const rtc8x_frame_params p, dev::V3 light, uint32_t spp,
             // two tentative collisions (a collision past the segment's end is looked up at the current
             // position, as the tracer does); a tracking segment stops at the first real one
             float tk[2], tl[2], u[2];
-            tk[0] = t + med.over(dev::neg_log_1m(rng.uni()), maj);
-            tk[1] = tk[0] + med.over(dev::neg_log_1m(rng.uni()), maj);
+            tk[0] = t + med.distance(dev::neg_log_1m(rng.uni()), maj);
+            tk[1] = tk[0] + med.distance(dev::neg_log_1m(rng.uni()), maj);
             u[0] = rng.uni();
             u[1] = rng.uni();
             tl[0] = tk[0] > t1 ? t : tk[0];

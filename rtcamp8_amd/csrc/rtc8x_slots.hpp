@@ -443,7 +443,7 @@ __device__ __forceinline__ void slots_body(ParamsPtr params, uint32_t W, uint32_
                         if (st == kWalking) {
                             const int r = w.visit(p.grid, med, sg.t, sg.t1, tau, mu, mem.regions);
                             if (r == kAdvanceCollision) {
-                                sg.t = sg.t + med.over(tau, mu);
+                                sg.t = sg.t + med.distance(tau, mu);
                                 st = kPending;
                             } else if (r == kAdvanceEnd) {
                                 st = kIdle;

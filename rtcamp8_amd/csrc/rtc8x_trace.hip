@@ -60,7 +60,7 @@ struct Seg<RTC8X_TRACKING_GLOBAL_MAJORANT> {
     }
     __device__ __forceinline__ bool advance(const rtc8x_grid&, const Medium& m, Pcg& rng, float& mu, const uint8_t*)
     {
-        t += m.over(neg_log_1m(rng.uni()), m.majorant);
+        t += m.distance(neg_log_1m(rng.uni()), m.majorant);
         if (t > t1) return false;
         mu = m.majorant;
         return true;
@@ -129,7 +129,7 @@ __device__ __forceinline__ void speculate_global(const rtc8x_grid& g, Medium& me
         ua[k] = 0.0f;
         st_after[k] = 0;
         if (!ended) {
-            t += med.over(neg_log_1m(r.uni()), med.majorant);
+            t += med.distance(neg_log_1m(r.uni()), med.majorant);
             if (t > sg.t1) {
                 ended = true;
                 st_end = r.state;
@@ -260,7 +260,7 @@ __device__ __forceinline__ void coop_segments(const rtc8x_grid& g, Medium& med, 
             const uint64_t st_step = r.state;  // after the step's draw
             const float ua = track ? r.uni() : 0.0f;
             const uint64_t st_after = r.state;
-            const float dj = med.over(neg_log_1m(u), maj);
+            const float dj = med.distance(neg_log_1m(u), maj);
             // t after collision j, summed in order; the segment ends at the first collision past t1
             float tj = INFINITY, run = t;
             uint32_t e = 64;
