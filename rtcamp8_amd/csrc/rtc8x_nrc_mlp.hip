@@ -554,7 +554,15 @@ __global__ __launch_bounds__(64 * WPB, WPB == 1 ? 1 : 3) void forward_kernel(con
 // The queries are the live ones of the inference: a workgroup takes every gridDim-th block of 512 slots,
 // compacts the slots with a query into a list and runs each full tile of it, so slots without a query cost
 // their flag only.
+//
+// A tile of fewer queries than kPlaneDirect gathers its corners from memory instead (hash_level_pairs, the same
+// sums): staging takes 66 us whatever the tile holds.  A 1080p image of 4 samples with 0.2, 1 and 2 % of its slots
+// live, one disc of them: 108, 110 and 127 us without this, 51, 69 and 119 with it (forward_kernel: 51, 89, 125).  A
+// line at 1,024 or 2,048 queries costs the full tiles registers (2,073,600 queries: 382 us, 447 and 594).
 constexpr uint32_t kPlaneWaves = 8, kPlaneThreads = 64 * kPlaneWaves, kPlaneQ = 8, kPlaneTile = kPlaneThreads * kPlaneQ;
+constexpr uint32_t kPlaneDirect = 512;
+constexpr uint32_t kPlaneScan = 4;  // blocks of slots whose flags are read together
+static_assert(kPlaneDirect % kPlaneThreads == 0 && kPlaneDirect <= kPlaneTile && kPlaneScan * kPlaneThreads <= kPlaneTile, "");
 typedef uint32_t u16v __attribute__((ext_vector_type(16)));
 
 template <typename T>
@@ -602,7 +610,8 @@ template <typename T>
 __global__ __launch_bounds__(kPlaneThreads) void forward_planes_kernel(const T* __restrict__ w, uint32_t L,
                                                                        const rtc8x_radiance_query* __restrict__ in, uint32_t n,
                                                                        float* __restrict__ out, const float* __restrict__ planes,
-                                                                       uint32_t p_grid, const HashGeom geom, const QueryMask mask)
+                                                                       const float* __restrict__ tables, uint32_t p_grid,
+                                                                       const HashGeom geom, const QueryMask mask)
 {
     using V = typename Vec8<T>::type;
     struct Net {
@@ -626,19 +635,39 @@ __global__ __launch_bounds__(kPlaneThreads) void forward_planes_kernel(const T* 
         __syncthreads();
         uint32_t count = 0;
         while (blk < blocks && count + kPlaneThreads <= kPlaneTile) {
-            const uint32_t s = blk * kPlaneThreads + tid;
-            const bool live = s < n && slot_has_query(mask, s);
-            const uint64_t b = __ballot(live);
+            // the flags of up to kPlaneScan blocks, all loads in flight together
+            const uint32_t take = count + kPlaneScan * kPlaneThreads <= kPlaneTile ? kPlaneScan : 1u;
+            bool live[kPlaneScan];
+            uint32_t total = 0, before[kPlaneScan];
+#pragma unroll
+            for (uint32_t j = 0; j < kPlaneScan; ++j) {
+                const uint64_t s = ((uint64_t)blk + (uint64_t)j * gridDim.x) * kPlaneThreads + tid;
+                live[j] = j < take && s < n;
+                if (mask.terms) {
+                    const uint32_t at = live[j] ? (uint32_t)s : 0u, k = at / mask.q_stride, i = at - k * mask.q_stride;
+                    const uint32_t flag = mask.terms[(size_t)k * mask.npx + min(i, mask.npx - 1u)].has_query;
+                    live[j] = live[j] && i < mask.npx && (flag & 1u) != 0u;
+                }
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < kPlaneScan; ++j) {
+                const uint64_t b = __ballot(live[j]);
+                before[j] = total + (uint32_t)__popcll(b & ((1ull << lane) - 1ull));
+                total += (uint32_t)__popcll(b);
+            }
             uint32_t base = 0;
-            if (lane == 0 && b) base = atomicAdd(&listed, (uint32_t)__popcll(b));
+            if (lane == 0 && total) base = atomicAdd(&listed, total);
             base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
-            if (live) list[base + (uint32_t)__popcll(b & ((1ull << lane) - 1ull))] = s;
-            blk += gridDim.x;
+#pragma unroll
+            for (uint32_t j = 0; j < kPlaneScan; ++j)
+                if (live[j]) list[base + before[j]] = (blk + j * gridDim.x) * kPlaneThreads + tid;
+            blk += take * gridDim.x;
             __syncthreads();
             count = listed;
             __syncthreads();
         }
         if (count == 0) continue;
+        const bool direct = count < kPlaneDirect;  // uniform over the workgroup
         // query q of this lane: entry (q * waves + wave) * 64 + lane of the list
         float p[kPlaneQ][3];
         u16v feat[kPlaneQ];
@@ -647,7 +676,7 @@ __global__ __launch_bounds__(kPlaneThreads) void forward_planes_kernel(const T* 
             const uint32_t e = q * kPlaneThreads + tid;
             query_position01(in[list[min(e, count - 1u)]], p[q]);
         }
-        for (uint32_t lv = 0; lv < kHashLevels; ++lv) {
+        for (uint32_t lv = 0; lv < kHashLevels && !direct; ++lv) {
             const uint32_t first = geom.offset[lv] / 2u, entries = level_entries(geom, lv, p_grid);
             float lo[kPlaneQ];
 #pragma unroll
@@ -687,10 +716,21 @@ __global__ __launch_bounds__(kPlaneThreads) void forward_planes_kernel(const T* 
             if (q * kPlaneThreads + wave * 64u >= count) continue;
             const uint32_t s = list[min(e, count - 1u)];
             T* row = &A[lane * kActStride];
+            if (q < kPlaneDirect / kPlaneThreads && direct) {
+                float pos[3];
+                query_position01(in[s], pos);
+#pragma unroll 1
+                for (uint32_t lv = 0; lv < kHashLevels; ++lv) {
+                    const float2 a = hash_level_pairs(pos, tables, geom, lv);
+                    row[2 * lv] = (T)a.x;
+                    row[2 * lv + 1] = (T)a.y;
+                }
+            } else {
 #pragma unroll
-            for (uint32_t j = 0; j < 4; ++j) {
-                const uint4 v = make_uint4(feat[q][4 * j], feat[q][4 * j + 1], feat[q][4 * j + 2], feat[q][4 * j + 3]);
-                *reinterpret_cast<uint4*>(&row[8 * j]) = v;
+                for (uint32_t j = 0; j < 4; ++j) {
+                    const uint4 v = make_uint4(feat[q][4 * j], feat[q][4 * j + 1], feat[q][4 * j + 2], feat[q][4 * j + 3]);
+                    *reinterpret_cast<uint4*>(&row[8 * j]) = v;
+                }
             }
             {
                 float t[32];
@@ -1441,7 +1481,8 @@ hipError_t launch_forward_enc(rtc8x_nrc* h, bool train, const void* w, const flo
 // queries costs a workgroup 66 us for staging the 32 planes, however few queries it holds, and 31 us per 1,024
 // for the gathers and the network; the direct kernel takes 52 us for 131,072 queries, 102 for 262,144 and 797
 // for 2,073,600, this one 75, 94 and 386.  With a mask the number of live slots is not known here: the line lies
-// where a twelfth of them break even.
+// where this kernel is the faster one from 0.2 % of them on (with none, reading their flags takes it 33 us and the
+// direct kernel 28).
 template <typename T>
 hipError_t launch_planes(rtc8x_nrc* h, hipStream_t s, const float* in, uint32_t n, float* out, const nrc::QueryMask& mask)
 {
@@ -1453,7 +1494,7 @@ hipError_t launch_planes(rtc8x_nrc* h, hipStream_t s, const float* in, uint32_t 
     const uint32_t blocks = (n + nrc::kPlaneThreads - 1) / nrc::kPlaneThreads;
     hipLaunchKernelGGL((nrc::forward_planes_kernel<T>), dim3(std::min<uint32_t>(blocks, (uint32_t)cus)), dim3(nrc::kPlaneThreads),
                        0, s, (const T*)h->winf, h->L, (const rtc8x_radiance_query*)in, n, out, (const float*)h->grid_planes,
-                       h->P_grid, h->geom, mask);
+                       (const float*)h->grid_inf, h->P_grid, h->geom, mask);
     return hipGetLastError();
 }
 constexpr uint32_t kPlanesMin = 163840, kPlanesMinMasked = 1u << 21;

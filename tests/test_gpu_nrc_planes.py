@@ -92,3 +92,47 @@ def test_masked_slots(live):
     assert np.array_equal(got[on], ref[on])
     assert (got[~on] == 7).all()
     c.finalize()
+
+
+@pytest.mark.parametrize("precision", [_abi.NRC_FP16, _abi.NRC_BF16])
+@pytest.mark.parametrize("live", ["one", "0.3 %", "a disc", "511 and 512"])
+def test_tiles_of_few_queries(live, precision):
+    """Tiles below and at the line under which corners are gathered from memory: the bits of the whole batch."""
+    from rtcamp8_amd.device import DeviceBuffer
+    from rtcamp8_amd.nrc import round_up
+
+    w, h, k = 1024, 640, 4
+    npx = w * h
+    stride = round_up(npx, 128)
+    n = stride * k
+    assert n >= MIN_MASKED
+    c = _cache(precision, layers=3)
+    dq = DeviceBuffer.from_array(_queries(n, 4))
+    flags = np.zeros((k, npx), bool)
+    rng = np.random.default_rng(10)
+    if live == "one":
+        flags[2, npx - 1] = True
+    elif live == "0.3 %":
+        flags = rng.random((k, npx)) < 0.003
+    elif live == "a disc":
+        y, x = np.divmod(np.arange(npx), w)
+        flags[:] = (x - 700) ** 2 + (y - 300) ** 2 < 90 ** 2
+    else:  # whole blocks of 512 slots, and blocks with one slot less
+        flags[0, : 512 * 256] = True
+        flags[0, ::1024] = False
+    terms = np.zeros((k * npx, 4), np.uint32)
+    terms[:, 3] = flags.reshape(-1) | 0x300
+    dt = DeviceBuffer.from_array(terms)
+    out = DeviceBuffer.from_array(np.full(3 * n, 7, np.uint32))
+    p = _abi.FrameParams()
+    p.image_width, p.image_height = w, h
+    p.nrc.num_samples = k
+    p.nrc.inference_queries, p.nrc.inferred_radiance, p.nrc.inference_terminals = dq.ptr, out.ptr, dt.ptr
+    c.infer_render(None, p)
+    got = out.download(np.uint32, 3 * n).reshape(k, stride, 3)
+    ref = _in_pieces(c, dq, n).reshape(k, stride, 3)
+    on = np.zeros((k, stride), bool)
+    on[:, :npx] = flags
+    assert on.any() and np.array_equal(got[on], ref[on])
+    assert (got[~on] == 7).all()
+    c.finalize()
