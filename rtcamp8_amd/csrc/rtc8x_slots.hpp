@@ -62,8 +62,8 @@ static_assert(RTC8X_MAX_REGIONS <= 1u << kIdxBits && kHardMaxPathLength < 1u << 
 
 constexpr uint32_t kDealt = 8;          // pixels of a workgroup's turn when they are dealt out
 constexpr uint32_t kLdsBytes = 163840;  // of a CU
-// REGION_BYTES: room for the region table (local majorants)
-template <int ENTRY, int TRACKING, uint32_t REGION_BYTES>
+// REGION_BYTES: room for the region table (local majorants); SLOTS: at most this many
+template <int ENTRY, int TRACKING, uint32_t REGION_BYTES, uint32_t SLOTS>
 struct SlotLayout {
     static constexpr bool kLocal = TRACKING == RTC8X_TRACKING_LOCAL_MAJORANT;
     static constexpr bool kNrc = ENTRY == RTC8X_ENTRY_PATH_TRACE_WITH_NRC;
@@ -73,12 +73,12 @@ struct SlotLayout {
     static constexpr uint32_t kSpread = kLocal ? kTau + 4 : kCommonFields;
     static constexpr uint32_t kFields = kSpread + (kNrc ? 2u : 0u);
     static constexpr uint32_t kFit = (kLdsBytes - REGION_BYTES - 4096u) / (4u * kFields) & ~63u;
-    static constexpr uint32_t kSlots = kFit < 1280u ? kFit : 1280u;
+    static constexpr uint32_t kSlots = kFit < SLOTS ? kFit : SLOTS;
 };
 
-template <int ENTRY, int TRACKING, uint32_t REGION_BYTES, uint32_t WAVES>
+template <int ENTRY, int TRACKING, uint32_t REGION_BYTES, uint32_t WAVES, uint32_t SLOTS>
 struct SlotMem {
-    using Lay = SlotLayout<ENTRY, TRACKING, REGION_BYTES>;
+    using Lay = SlotLayout<ENTRY, TRACKING, REGION_BYTES, SLOTS>;
     uint32_t f[Lay::kFields][Lay::kSlots];
     uint32_t ready[kWorkKinds][64];  // bit b of word w: slot 64 b + w
     int32_t count[8];                // slots ready per kind (a hint: the masks decide)
@@ -206,12 +206,12 @@ typedef const __attribute__((address_space(4))) rtc8x_frame_params* ParamsPtr;
 
 // One image by workgroup wg of its wgs; helper: a workgroup of another image of the batch, which takes pixels
 // from this one's work counter only.
-template <int ENTRY, int TRACKING, uint32_t REGION_BYTES, uint32_t WAVES>
+template <int ENTRY, int TRACKING, uint32_t REGION_BYTES, uint32_t WAVES, uint32_t SLOTS>
 __device__ __forceinline__ void slots_body(ParamsPtr params, uint32_t W, uint32_t H, uint32_t num_samples, uint32_t ctr,
                                            uint32_t wg, uint32_t wgs, bool helper,
-                                           SlotMem<ENTRY, TRACKING, REGION_BYTES, WAVES>& mem)
+                                           SlotMem<ENTRY, TRACKING, REGION_BYTES, WAVES, SLOTS>& mem)
 {
-    using Lay = SlotLayout<ENTRY, TRACKING, REGION_BYTES>;
+    using Lay = SlotLayout<ENTRY, TRACKING, REGION_BYTES, SLOTS>;
     constexpr bool kLocal = Lay::kLocal, kNrc = Lay::kNrc;
     const rtc8x_frame_params& p = *(const rtc8x_frame_params*)params;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
@@ -832,13 +832,13 @@ __device__ __forceinline__ void slots_body(ParamsPtr params, uint32_t W, uint32_
     }
 }
 
-template <int ENTRY, int TRACKING, uint32_t REGION_BYTES, uint32_t WAVES>
+template <int ENTRY, int TRACKING, uint32_t REGION_BYTES, uint32_t WAVES, uint32_t SLOTS>
 __global__ __launch_bounds__(64 * WAVES) void slots_kernel(const rtc8x_frame_params p, uint32_t W, uint32_t H,
                                                            uint32_t num_samples, uint32_t ctr)
 {
     (void)p;  // the first kernel argument, read through the argument segment
-    __shared__ SlotMem<ENTRY, TRACKING, REGION_BYTES, WAVES> mem;
-    slots_body<ENTRY, TRACKING, REGION_BYTES, WAVES>((ParamsPtr)__builtin_amdgcn_kernarg_segment_ptr(), W, H, num_samples, ctr,
+    __shared__ SlotMem<ENTRY, TRACKING, REGION_BYTES, WAVES, SLOTS> mem;
+    slots_body<ENTRY, TRACKING, REGION_BYTES, WAVES, SLOTS>((ParamsPtr)__builtin_amdgcn_kernarg_segment_ptr(), W, H, num_samples, ctr,
                                                      blockIdx.x, gridDim.x, false, mem);
 }
 
@@ -853,17 +853,17 @@ struct BatchArgs {
     uint32_t num_samples[kMaxBatch];
 };
 
-template <int ENTRY, int TRACKING, uint32_t REGION_BYTES, uint32_t WAVES>
+template <int ENTRY, int TRACKING, uint32_t REGION_BYTES, uint32_t WAVES, uint32_t SLOTS>
 __global__ __launch_bounds__(64 * WAVES) void slots_batch_kernel(const BatchArgs b)
 {
-    __shared__ SlotMem<ENTRY, TRACKING, REGION_BYTES, WAVES> mem;
+    __shared__ SlotMem<ENTRY, TRACKING, REGION_BYTES, WAVES, SLOTS> mem;
     uint32_t first = 0;
     while (first + 1 < b.count && blockIdx.x >= b.wg_end[first]) ++first;
     for (uint32_t k = 0; k < b.count; ++k) {
         const uint32_t inst = first + k < b.count ? first + k : first + k - b.count;
         const uint32_t wg0 = inst ? b.wg_end[inst - 1] : 0u;
         const rtc8x_frame_params* pp = b.params + inst;
-        slots_body<ENTRY, TRACKING, REGION_BYTES, WAVES>((ParamsPtr)(uint64_t)pp, pp->image_width, pp->image_height,
+        slots_body<ENTRY, TRACKING, REGION_BYTES, WAVES, SLOTS>((ParamsPtr)(uint64_t)pp, pp->image_width, pp->image_height,
                                                          b.num_samples[inst], b.ctr + inst, blockIdx.x - wg0,
                                                          b.wg_end[inst] - wg0, k != 0, mem);
         __syncthreads();  // the LDS is free for the next instance

@@ -1305,6 +1305,11 @@ hipError_t launch(const rtc8x_frame_params& p, const uint32_t* offsets, uint32_t
 // the others would only look for work (256 x 256, 4 samples: 0.71 ms with 8, 0.74 with 6, 0.75 with 12, 0.85
 // with 16 wavefronts).
 constexpr uint32_t kSlotWaves = 16, kSlotWavesFew = 8;
+// Such an image also needs no more than its 512 slots a CU (and what its tiles are padded by).  That leaves LDS and
+// registers to kernels of another stream: in a 256 x 256 cache-rendered frame the last training step's scatter, begun
+// with the trace, lasted the trace's 384 us and now 108, and its reduction and optimiser no longer follow the trace
+// (frame 1.374 -> 1.363 ms).
+constexpr uint32_t kMostSlots = 1280, kFewSlots = 640;
 inline bool few_paths(uint64_t pixels, uint32_t workgroups) { return pixels <= 64ull * kSlotWavesFew * workgroups; }
 inline uint32_t region_bytes(const rtc8x_grid& g)
 {
@@ -1320,9 +1325,12 @@ hipError_t launch_slots(const rtc8x_frame_params& p, uint32_t num_samples, hipSt
     e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(reset_counter_kernel, dim3(1), dim3(1), 0, stream, ctr);
-    const uint32_t waves = few_paths((uint64_t)p.image_width * p.image_height, (uint32_t)cus) ? kSlotWavesFew : kSlotWaves;
-    hipLaunchKernelGGL((slots_kernel<ENTRY, TRACKING, REGION_BYTES, kSlotWaves>), dim3((uint32_t)cus), dim3(64 * waves), 0,
-                       stream, p, p.image_width, p.image_height, num_samples, ctr);
+    if (few_paths((uint64_t)p.image_width * p.image_height, (uint32_t)cus))
+        hipLaunchKernelGGL((slots_kernel<ENTRY, TRACKING, REGION_BYTES, kSlotWaves, kFewSlots>), dim3((uint32_t)cus),
+                           dim3(64 * kSlotWavesFew), 0, stream, p, p.image_width, p.image_height, num_samples, ctr);
+    else
+        hipLaunchKernelGGL((slots_kernel<ENTRY, TRACKING, REGION_BYTES, kSlotWaves, kMostSlots>), dim3((uint32_t)cus),
+                           dim3(64 * kSlotWaves), 0, stream, p, p.image_width, p.image_height, num_samples, ctr);
     return hipGetLastError();
 }
 
@@ -1371,7 +1379,7 @@ hipError_t launch_batch(const rtc8x_frame_params* params, const rtc8x_frame_para
         few &= few_paths((uint64_t)params[i].image_width * params[i].image_height, end - begin);
     }
     hipLaunchKernelGGL(reset_counters_kernel, dim3(1), dim3(kMaxBatch), 0, stream, ctr, count);
-    hipLaunchKernelGGL((slots_batch_kernel<ENTRY, TRACKING, REGION_BYTES, kSlotWaves>), dim3(end),
+    hipLaunchKernelGGL((slots_batch_kernel<ENTRY, TRACKING, REGION_BYTES, kSlotWaves, kMostSlots>), dim3(end),
                        dim3(64 * (few ? kSlotWavesFew : kSlotWaves)), 0, stream, b);
     return hipGetLastError();
 }

@@ -44,3 +44,12 @@ def test_large_region_table(region_cells):
 def test_majorant_below_the_fast_divisions_range(tracking):
     _check(trace_parity_case("dense128", width=40, height=24, spp=2, tracking=tracking, fbm_resolution=64,
                              density_coeff=2.0 ** -42), 40 * 24, 2)
+
+
+@pytest.mark.parametrize("tracking", [0, 1])
+@pytest.mark.parametrize("width,height", [(362, 362), (364, 361), (14563, 9), (16384, 8)])
+def test_at_the_line_of_few_paths(width, height, tracking):
+    """Just below, above and at 512 pixels a workgroup on 256 CUs; and below it with rows that its tiles pad to
+    more than the slots of the small variant."""
+    _check(trace_parity_case("dense128", width=width, height=height, spp=1, tracking=tracking, fbm_resolution=64,
+                             env_kind="constant", max_path_length=12), width * height, 1)
