@@ -86,6 +86,11 @@ struct rtc8x_grid;
 rtc8x_status rtc8x_copy_async(void* dst, const void* src, size_t bytes, void* stream);
 rtc8x_status rtc8x_gather_probe(void* stream, const struct rtc8x_grid* grid, uint32_t threads, uint32_t steps,
                                 uint32_t width, uint32_t waves_per_simd, uint32_t seed, float* out);
+/* rtc8x_math_probe: the trackers' short forms of single-precision functions beside the functions themselves, for n
+ *   operands; device arrays.  op 0: -log(1 - a) of a number a = k 2^-23 in [0, 1), as the trackers draw it; op 1:
+ *   the same by rtc8x_logf; op 2: a density a over a majorant b in [2^-40, 2^40]; op 3: an optical depth a over
+ *   such a majorant.  b may be NULL for op 0 and 1. */
+rtc8x_status rtc8x_math_probe(void* stream, int32_t op, uint32_t n, const float* a, const float* b, float* out);
 
 struct rtc8x_frame_params;
 /*

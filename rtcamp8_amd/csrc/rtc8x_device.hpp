@@ -48,7 +48,8 @@ __device__ __forceinline__ V3 normalize(V3 v)
 // a / b, correctly rounded as the IEEE division is, where no intermediate leaves the normal range: the
 // division's own sequence of corrections without its scaling and special cases (8 instructions against 14).
 // Equal to a / b in 2^32 trials over |a| in [2^-85, 2^40], b in [2^-40, 2^40], mantissas at both ends
-// included.  A smaller |a| can miss the last bit of a quotient far below everything it is compared with.
+// included; -0 gives +0.  A smaller |a| can miss the last bit of a quotient far below everything it is compared
+// with.
 __device__ __forceinline__ float div_normal(float a, float b)
 {
     float r = __builtin_amdgcn_rcpf(b);

@@ -63,6 +63,20 @@ __global__ void gather_probe_kernel(const rtc8x_grid g, uint32_t steps, uint32_t
     out[tid] = acc;
 }
 
+__global__ __launch_bounds__(256) void math_probe_kernel(int32_t op, uint32_t n, const float* __restrict__ a,
+                                                         const float* __restrict__ b, float* __restrict__ out)
+{
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= n) return;
+    dev::Medium med{};
+    med.normal = true;
+    const float x = a[i];
+    out[i] = op == 0   ? dev::neg_log_1m(x)
+             : op == 1 ? -rtc8x_logf(1.0f - x)
+             : op == 2 ? med.over(x, b[i])
+                       : med.distance(x, b[i]);
+}
+
 // The tracer's stepping pattern with its shading taken out, as a persistent launch like the tracer's:
 // lanes take pixels in 8x8 tiles from a work counter (one atomic per wavefront, the tiles wrapping around
 // the image) and trace every one of a pixel's `spp` paths before the next: a jittered camera ray
@@ -310,6 +324,18 @@ try {
     return RTC8X_OK;
 }
 RTC8X_CATCH_ALL("rtc8x_gather_probe")
+
+extern "C" rtc8x_status rtc8x_math_probe(void* stream, int32_t op, uint32_t n, const float* a, const float* b, float* out)
+try {
+    RTC8X_REQUIRE(op >= 0 && op <= 3, "rtc8x_math_probe: unknown op %d", (int)op);
+    if (n == 0) return RTC8X_OK;
+    RTC8X_REQUIRE(a && out && (op < 2 || b), "rtc8x_math_probe: NULL pointer");
+    hipLaunchKernelGGL(math_probe_kernel, dim3((uint32_t)(((uint64_t)n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, op, n, a,
+                       b, out);
+    RTC8X_HIP(hipGetLastError());
+    return RTC8X_OK;
+}
+RTC8X_CATCH_ALL("rtc8x_math_probe")
 
 extern "C" rtc8x_status rtc8x_march_probe(void* stream, const rtc8x_frame_params* params, const float light_dir[3],
                                           uint32_t spp, uint32_t budget, uint32_t waves_per_simd, uint64_t* stats)

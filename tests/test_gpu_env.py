@@ -194,3 +194,37 @@ def test_alias_tables_equal_the_serial_method(w, h):
         assert env.alias_integral == np.float32(total)
     finally:
         call("rtc8x_env_release", C.byref(env))
+
+
+@pytest.mark.parametrize("h", [9831, 16384])
+def test_alias_tables_of_the_tallest_textures(h):
+    """Heights whose table of rows takes more than 96 KB of LDS, up to all of a CU's: that table and some rows'."""
+    import torch
+
+    from rtcamp8_amd import _abi
+    from rtcamp8_amd._lib import call
+    from rtcamp8_amd.device import download_ptr
+
+    w = 8193
+    g = torch.Generator(device="cuda").manual_seed(h)
+    tex = torch.zeros(h, w, 4, device="cuda")
+    tex[..., :3] = torch.rand(h, w, 1, generator=g, device="cuda") ** 4 * torch.rand(h, 1, 1, generator=g, device="cuda") ** 3
+    torch.cuda.synchronize()
+    env = _abi.EnvLight()
+    env.kind, env.width, env.height, env.texels = _abi.ENV_LATLONG, w, h, tex.data_ptr()
+    call("rtc8x_env_build_sampler", C.byref(env), None)
+    try:
+        weights = download_ptr(env.alias_weights, np.float32, w * h).reshape(h, w)
+        sums = np.zeros(h)
+        for x in range(w):  # each row's sum in texel order
+            sums += weights[:, x]
+        total, second, first = _vose([float(x) for x in sums])
+        rows = download_ptr(env.alias_rows, np.uint32, 2 * h).reshape(h, 2)
+        assert np.array_equal(second, rows[:, 0]) and np.array_equal(first.view(np.uint32), rows[:, 1])
+        assert env.alias_integral == np.float32(total)
+        for y in (0, 1, h // 2, h - 1):
+            cols = download_ptr(env.alias_cols + 8 * y * w, np.uint32, 2 * w).reshape(w, 2)
+            _, second, first = _vose([float(x) for x in weights[y]])
+            assert np.array_equal(second, cols[:, 0]) and np.array_equal(first.view(np.uint32), cols[:, 1]), y
+    finally:
+        call("rtc8x_env_release", C.byref(env))
