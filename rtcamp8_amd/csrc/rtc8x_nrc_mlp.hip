@@ -1479,8 +1479,9 @@ hipError_t launch_forward_enc(rtc8x_nrc* h, bool train, const void* w, const flo
 
 // Inference of n slots by forward_planes_kernel, for 16-bit networks with the hash grid.  A tile of 4,096
 // queries costs a workgroup 66 us for staging the 32 planes, however few queries it holds, and 31 us per 1,024
-// for the gathers and the network; the direct kernel takes 52 us for 131,072 queries, 102 for 262,144 and 797
-// for 2,073,600, this one 75, 94 and 386.  With a mask the number of live slots is not known here: the line lies
+// for the gathers and the network.  The direct kernel's time jumps where its workgroups of 256 no longer fit the
+// device at once, three a CU: 196,608 queries take it 73 us and 197,000 88 (eight layers 90 and 107), this one 82 and
+// 82 (106 and 106); 2,073,600 take 698 and 382.  With a mask the number of live slots is not known here: the line lies
 // where this kernel is the faster one from 0.2 % of them on (with none, reading their flags takes it 33 us and the
 // direct kernel 28).
 template <typename T>
@@ -1497,7 +1498,7 @@ hipError_t launch_planes(rtc8x_nrc* h, hipStream_t s, const float* in, uint32_t 
                        (const float*)h->grid_inf, h->P_grid, h->geom, mask);
     return hipGetLastError();
 }
-constexpr uint32_t kPlanesMin = 163840, kPlanesMinMasked = 1u << 21;
+constexpr uint32_t kPlanesMin = 3 * 256 * 256 + 256, kPlanesMinMasked = 1u << 21;
 
 // train: the working weights and the FP32 master tables; inference: the EMA weights and tables
 template <typename T>

@@ -136,3 +136,16 @@ def test_tiles_of_few_queries(live, precision):
     assert on.any() and np.array_equal(got[on], ref[on])
     assert (got[~on] == 7).all()
     c.finalize()
+
+
+@pytest.mark.parametrize("n", [196608 + 255, 196608 + 256, 196608 + 511])
+def test_at_the_line(n):
+    """The last batch of the direct kernel and the first ones of the planes."""
+    from rtcamp8_amd.device import DeviceBuffer
+
+    c = _cache(_abi.NRC_FP16, layers=8)
+    dq = DeviceBuffer.from_array(_queries(n, n))
+    out = DeviceBuffer.zeros(12 * n)
+    c.infer(None, dq.ptr, n, out.ptr)
+    assert np.array_equal(out.download(np.uint32, 3 * n), _in_pieces(c, dq, n))
+    c.finalize()
