@@ -118,9 +118,10 @@ def saturated_leg(args, stream, tracking: int) -> dict:
 
 def traffic_from_profiles(kernel: str, workload: str):
     """HBM bytes per launch from the committed rocprofv3 --pmc summary (profiles/<kernel>_<workload>_hbm.json),
-    if there is one."""
+    if there is one; says so if there is none."""
     f = ROOT / "profiles" / f"{kernel}_{workload}_hbm.json"
     if not f.exists():
+        print(f"[bench] no counter summary {f.relative_to(ROOT)}: traffic is not reported", file=sys.stderr, flush=True)
         return None
     try:
         return float(json.loads(f.read_text())["hbm_bytes_per_launch"])
@@ -387,15 +388,16 @@ def nrc_render_leg(scene, steps: int, stream):
 
 
 def latency_roofline(scene, params, lookups_per_launch: float, lookups_per_path: float, trace_lookups_per_s: float,
-                     paths_per_s: float, waves=(3, 4)):
-    """Memory-latency roofline of the tracer's density lookups: the march probe (rtc8x_march_probe) walks
+                     paths_per_s: float, waves=(4, 3)):
+    """A reference rate for the tracer's density lookups: the march probe (rtc8x_march_probe) walks
     the tracer's own stepping pattern on this frame -- persistent lanes taking the frame's pixels in 8x8
     tiles, the same camera rays and PCG states, delta tracking at the majorant's spacing with two tentative
     collisions looked up together, a ratio-tracked shadow segment towards the sun and a phase sample at
     every real collision -- with none of the tracer's vertex shading, and every lane stops at the same
-    lookup budget (as many lookups in all as one traced frame) so the launch has no tail.  The reference
-    point is the tracer's occupancy (3 waves per SIMD, registers allotted as for the tracer), 4 waves
-    beside it; the gather probe (random positions of random leaves, no coherence) is reported too."""
+    lookup budget (as many lookups in all as one traced frame) so the launch has no tail.  It is taken at the
+    tracer's occupancy (4 waves per SIMD), with 3 waves beside it.  It is no bound: its lanes keep their paths,
+    where the tracer's wavefronts draw full chunks of work from path slots.  The gather probe (random positions
+    of random leaves, no coherence) is reported too."""
     from rtcamp8_amd import scene as sc
     from rtcamp8_amd._lib import call
     from rtcamp8_amd.device import DeviceBuffer, EventTimer, device_cus
@@ -602,8 +604,8 @@ def global_majorant_leg(scene, pt, spp: int, steps: int, stream) -> dict:
                                                c["lookups"] / sum(kernel_ms) * 1e3, out["paths_per_s"])
     pt.stats.fill(0)
     print(f"[bench] global-majorant tracking: {ms:.2f} ms per frame, {out['path_vertices_per_s']:.3g} vertices/s, "
-          f"{out['lookups_per_path']:.1f} lookups/path, {out['latency_roofline']['paths_frac']:.2f} of its latency "
-          "roofline", file=sys.stderr, flush=True)
+          f"{out['lookups_per_path']:.1f} lookups/path, {out['latency_roofline']['paths_frac']:.2f} of the march "
+          "probe's rate", file=sys.stderr, flush=True)
     return out
 
 
@@ -720,12 +722,12 @@ def main() -> int:
     result["lookups_per_path"] = c["lookups"] / max(c["paths"], 1)
     if args.legs != "all":
         return finish(args, result, timers, pt, scene, stream, network_only=args.legs == "network")
-    waves = (3, 4)
+    waves = (4, 3)
     lat = latency_roofline(scene, params, lookups_per_launch, c["lookups"] / max(c["paths"], 1),
                            c["lookups"] / sum(kernel_ms) * 1e3, c["paths"] / wall, waves=waves)
     result["latency_roofline"] = lat
-    print(f"[bench] latency roofline ({lat['tracking']} tracking): march probe {lat['lookups_per_s_3waves']:.3g} "
-          f"lookups/s at 3 waves/SIMD ({lat[f'lookups_per_s_{waves[1]}waves']:.3g} at {waves[1]}); trace at "
+    print(f"[bench] reference rate ({lat['tracking']} tracking): march probe {lat[f'lookups_per_s_{waves[0]}waves']:.3g} "
+          f"lookups/s at {waves[0]} waves/SIMD ({lat[f'lookups_per_s_{waves[1]}waves']:.3g} at {waves[1]}); trace at "
           f"{lat['frac']:.2f} of it, paths at {lat['paths_frac']:.2f}", file=sys.stderr, flush=True)
     if tracking == _abi.TRACKING_LOCAL_MAJORANT:
         print("[bench] global-majorant leg ...", file=sys.stderr, flush=True)

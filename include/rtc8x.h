@@ -76,9 +76,9 @@ rtc8x_status rtc8x_stream_wait_event(void* stream, void* event);
 /* Measurement kernels (no counterpart in the reference).
  * rtc8x_copy_async: device-to-device copy by a plain 16-byte-per-lane kernel on `stream` (dst, src and
  *   bytes 16-byte aligned).  It reads and writes exactly `bytes` each, which calibrates HBM byte counters.
- * rtc8x_gather_probe: the memory-latency roofline of density lookups.  `threads` lanes (a multiple of
+ * rtc8x_gather_probe: the rate of density lookups without coherence.  `threads` lanes (a multiple of
  *   256) each perform `steps` serially dependent steps of `width` (1, 2, 4) lookups issued together;
- *   a lookup is the tracer's trilinear lookup (leaf-map entry, then the 2x2x2 stencil's voxels) at a
+ *   a lookup is the tracer's trilinear lookup (a map entry, then the 2x2x2 stencil's voxels) at a
  *   random position inside a random leaf of the device grid `grid`.  Occupancy is pinned to
  *   `waves_per_simd` (2..8) waves per SIMD through an LDS reservation.  out[threads] receives a per-lane
  *   checksum. */
@@ -94,10 +94,10 @@ rtc8x_status rtc8x_math_probe(void* stream, int32_t op, uint32_t n, const float*
 
 struct rtc8x_frame_params;
 /*
- * rtc8x_march_probe: the memory-latency roofline of the tracer's own lookups (no counterpart in the
+ * rtc8x_march_probe: a reference rate for the tracer's own lookups (no counterpart in the
  * reference).  A persistent launch, `waves_per_simd` (2..4, set with dynamic LDS) 256-lane workgroups per
- * CU (registers allotted for 3 waves per SIMD, as the tracer's render entries have, up to 3, and for 4
- * at 4), whose lanes take the frame's pixels in 8x8 tiles from a work counter as the tracer's do (the
+ * CU (registers allotted for 3 waves per SIMD up to 3, and for 4, the tracer's own occupancy, at 4),
+ * whose lanes take the frame's pixels in 8x8 tiles from a work counter as the tracer's do (the
  * tiles wrapping around the image; a pixel's PCG state is read, never written) and trace `spp` paths per
  * pixel: jittered camera rays, delta tracking as params->tracking selects it (the global majorant's
  * spacing with two tentative collisions looked up together, or the local tracker's region walk over the
@@ -147,7 +147,8 @@ typedef struct rtc8x_grid {
     const uint32_t* upper_tables;        /* num_upper * 32768 entries */
     const uint32_t* lower_tables;        /* num_lower * 4096 entries */
     /* Device grids (from rtc8x_grid_build_fbm / rtc8x_grid_upload*) keep one float of padding after
-     * leaf_values and after tile_values: the tracer reads voxel pairs (z, z+1) without a bounds test. */
+     * leaf_values and after tile_values: lookups without bricks read voxel pairs (z, z+1) without a
+     * bounds test. */
     const float* leaf_values;            /* num_leaves * 512 voxel values */
     const float* tile_values;            /* tile_values[0] == background */
     const int32_t* leaf_origins;         /* num_leaves * 3 index-space origins (optional, may be NULL) */

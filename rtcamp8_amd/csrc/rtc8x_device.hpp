@@ -610,7 +610,7 @@ constexpr uint32_t kRegionBudget = 6;
 enum : int { kAdvanceEnd = 0, kAdvanceCollision = 1, kAdvanceBudget = 2 };
 
 // Local majorants over the grid's regions, the loops of track_local / ratio_local made resumable; the
-// region bytes come from `table` (a copy staged in LDS by the single-image kernel).
+// region bytes come from `table` (a copy staged in LDS).
 template <>
 struct Seg<RTC8X_TRACKING_LOCAL_MAJORANT> {
     V3 o, d;

@@ -1,7 +1,7 @@
 // rtc8x_measure.hip -- measurement kernels with no counterpart in the renderer: a plain copy (the
 // calibration of the HBM byte counters), dependent density lookups at random positions of the grid's
-// leaves, and the tracer's own stepping pattern with its shading taken out (the memory-latency roofline
-// of the tracer's lookups).
+// leaves, the tracer's own stepping pattern with its shading taken out (a reference rate for the tracer's
+// lookups), and the trackers' short math beside the functions it stands for.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -28,7 +28,7 @@ __device__ __forceinline__ uint32_t mix32(uint32_t h)
 }
 
 // Each lane performs `steps` steps of W density lookups.  A lookup is the tracer's own: the trilinear
-// stencil at a random position inside a random leaf, fetched in two rounds (leaf-map entries, then the
+// stencil at a random position inside a random leaf, fetched in two rounds (map entries, then the
 // voxels) by trilinear_batch, whose W lookups overlap.  The next step's positions depend on the values
 // read, so steps are serially dependent.
 template <uint32_t W>
@@ -92,8 +92,8 @@ __global__ __launch_bounds__(256) void math_probe_kernel(int32_t op, uint32_t n,
 __device__ uint32_t g_probe_counter;
 __global__ void reset_probe_kernel() { g_probe_counter = 0u; }
 
-// WAVES: the occupancy the registers are allotted for (3: 168 VGPRs, as the tracer's render entries; 4:
-// 128), the launch's own occupancy being set by the LDS reservation.
+// WAVES: the occupancy the registers are allotted for (3: 168 VGPRs; 4: 128, as the tracer's full-image
+// launches), the launch's own occupancy being set by the LDS reservation.
 template <int TRACKING, int WAVES>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES)))
 void march_probe_kernel(const rtc8x_frame_params p, dev::V3 light, uint32_t spp, uint32_t budget,

@@ -1,5 +1,5 @@
-// rtc8x_slots.hpp -- the full-image launches (PATH_TRACE and PATH_TRACE_WITH_NRC) as a scheduler of path
-// slots: renderer/gpu_kernels/optix_pathtracing_kernels.cu:31-448 for volume-only scenes.
+// rtc8x_slots.hpp -- the full-image launches (PATH_TRACE and PATH_TRACE_WITH_NRC), single and batched, as a
+// scheduler of path slots: renderer/gpu_kernels/optix_pathtracing_kernels.cu:31-448 for volume-only scenes.
 //
 // One persistent workgroup per CU keeps about a thousand paths ("slots") in LDS, one dword per field and
 // slot.  A slot is ready for exactly one kind of work -- a density lookup, a region walk, an escape, the end
@@ -10,8 +10,8 @@
 //
 // What bounds the tracer is VALU issue and, next to it, the latency of the lookups.  With a path per lane for
 // its whole life, 14 of 64 lanes did work per VALU instruction with the local majorants and 24 with the global
-// one, and a third of the time went to vertex events with a few lanes each; here it is 32 and 43, in 12 G
-// instead of 18-19 G instructions per frame.  512^3 cloud, 1080p, 16 samples: 35.3 -> 24.9 ms (local), 36.5
+// one, and a third of the time went to vertex events with a few lanes each; here it is 26 and 44, in 10.3 G
+// and 10.8 G instead of 18-19 G instructions per frame.  512^3 cloud, 1080p, 16 samples: 35.3 -> 24.9 ms (local), 36.5
 // -> 29.2 ms (global); dense 128^3 cloud, 256 x 256, 4 samples: 1.17 -> 0.71 ms; 203 x 117, 1 sample, with the
 // work order and tone map: 521 -> 271 us.
 //
