@@ -1,4 +1,4 @@
-"""The march probe (rtc8x_march_probe), the latency ceiling the bench compares the tracer with: both of its
+"""The march probe (rtc8x_march_probe), the reference rate the bench compares the tracer with: both of its
 walks run to their lookup budget, count paths, and replay the tracker they stand for (the local walk does
 the local tracker's few lookups per path, the global one the global tracker's many)."""
 import ctypes as C

@@ -10,7 +10,7 @@ from rtcamp8_amd import _abi
 
 pytestmark = pytest.mark.gpu
 
-MIN, MIN_MASKED, PIECE = 163840, 1 << 21, 100000
+MIN, MIN_MASKED, PIECE = 3 * 256 * 256 + 256, 1 << 21, 100000
 
 
 def _queries(n, seed):
@@ -138,7 +138,7 @@ def test_tiles_of_few_queries(live, precision):
     c.finalize()
 
 
-@pytest.mark.parametrize("n", [196608 + 255, 196608 + 256, 196608 + 511])
+@pytest.mark.parametrize("n", [MIN - 1, MIN, MIN + 255])
 def test_at_the_line(n):
     """The last batch of the direct kernel and the first ones of the planes."""
     from rtcamp8_amd.device import DeviceBuffer
